@@ -63,7 +63,8 @@ extern "C" {
 #define LLMOPT_ALGO_GENERIC 1 /* any shape and dtype; scalar dequant + fp32 dot */
 #define LLMOPT_ALGO_DECODE 2  /* MFMA skinny GEMM, M <= 64 */
 #define LLMOPT_ALGO_PREFILL 3 /* MFMA GEMM with weight tiles dequantized into LDS */
-#define LLMOPT_ALGO_DENSE 4   /* the weight dequantized into the workspace, then hipBLASLt */
+#define LLMOPT_ALGO_DENSE 4   /* the weight dequantized into the workspace, then hipBLASLt; fp32 activations
+                                 of 65 tokens up: what AUTO runs (the same workspace is asked for) */
 
 /* ABI version of the loaded library (LLMOPT_QLINEAR_ABI_VERSION). */
 int llmopt_q_abi_version(void);
@@ -118,9 +119,10 @@ size_t llmopt_q_linear_workspace(int64_t M, int64_t N, int64_t K, int bits, int 
  * llmopt_q_linear_workspace for an activation dtype: the same for LLMOPT_DTYPE_BF16 / F16; for
  * LLMOPT_DTYPE_F32 the bytes of the fp32 path -- each activation split exactly into three bf16
  * pieces (3 * M * K * 2 bytes), the decode kernels' fp32 sums of a chunk of up to 21 tokens
- * (3 * chunk * N * 4) and their K-split partial sums; from 65 tokens, the two-pass path's fp32
- * llmopt_q_linear_dense_workspace bytes (or the pieces', if larger). With less, fp32 runs on the
- * generic kernel.
+ * (3 * chunk * N * 4) and their K-split partial sums, or, past one such chunk, the fp32 GEMM's pieces
+ * and partial sums if larger; from 65 tokens, the two-pass path's fp32
+ * llmopt_q_linear_dense_workspace bytes (or the pieces', if larger), for the shapes that the GEMM
+ * does not take. With less, fp32 runs on the decode kernels or the generic kernel.
  * Sizes the workspace of QuantLinear.forward with compute_dtype float32
  * (src/llmopt/quantization/quant_linear.py:93-113), the reference engine's quantized model
  * (engine/llm_engine.py:258-264).

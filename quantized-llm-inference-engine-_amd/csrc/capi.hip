@@ -2,8 +2,9 @@
 //
 // Validates arguments the way the reference's torch code would reject them, fills the
 // kernel argument block and picks the kernel: the decode kernels for M <= 32, the MFMA
-// register-dequant GEMM (split over K on small grids) above, from 1024 tokens (65 with fp32
-// activations) the weight dequantized into the workspace and hipBLASLt's dense GEMM, the
+// register-dequant GEMM (split over K on small grids) above, from 1024 tokens the weight
+// dequantized into the workspace and hipBLASLt's dense GEMM, for fp32 activations past one decode pass
+// the GEMM over exact bf16 pieces (the dense product for the shapes that it does not take), the
 // LDS-dequant GEMM for the shapes the register-dequant one does not take, and the generic kernel
 // for shapes, alignments or dtypes the fast kernels do not take. Error text is kept per host
 // thread.
@@ -199,6 +200,15 @@ int run_linear(const void* x, int64_t M, int64_t K, int64_t ldx, const void* qwe
     return hip_status(llmopt::launch_swiglu_combine(t, N, y, ldy, M, N, act_dtype, s), "swiglu launch");
   }
 
+  if (act_dtype == LLMOPT_DTYPE_F32 && M >= llmopt::f32_gemm_min_tokens(a.group) &&
+      (algo == LLMOPT_ALGO_AUTO ||
+       (algo == LLMOPT_ALGO_DENSE && dense_first(M, N, K, act_dtype, a.workspace, a.workspace_bytes)))) {
+    // fp32 activations past one decode pass: the GEMM over exact bf16 pieces, which also stands in
+    // for the dense product where that would run.
+    err = llmopt::launch_linear_f32_gemm(a, s, &fits);
+    if (fits) return hip_status(err, "fp32 linear");
+  }
+
   if (algo == LLMOPT_ALGO_DENSE || (algo == LLMOPT_ALGO_AUTO && dense_first(M, N, K, act_dtype, a.workspace,
                                                                                a.workspace_bytes))) {
     // Long batches: the weight dequantized into the workspace, then hipBLASLt's dense GEMM.
@@ -387,7 +397,10 @@ size_t llmopt_q_linear_workspace(int64_t M, int64_t N, int64_t K, int bits, int 
 size_t llmopt_q_linear_workspace_ex(int64_t M, int64_t N, int64_t K, int bits, int group_size, int act_dtype) {
   if (act_dtype != LLMOPT_DTYPE_F32) return llmopt_q_linear_workspace(M, N, K, bits, group_size);
   if (M <= 0 || N <= 0 || K <= 0 || bits < 1 || bits > 8) return 0;
-  const size_t pieces = llmopt::f32_workspace_bytes(M, N, K, group_size <= 0 ? K : group_size, bits);
+  const int64_t group = group_size <= 0 ? K : group_size;
+  size_t pieces = llmopt::f32_workspace_bytes(M, N, K, group, bits);
+  if (M >= llmopt::f32_gemm_min_tokens(group))
+    pieces = std::max(pieces, llmopt::f32_gemm_workspace_bytes(M, N, K, group));
   if (M < llmopt::dense_min_tokens(LLMOPT_DTYPE_F32)) return pieces;
   return std::max(pieces, llmopt::dense_workspace_bytes(N, K, LLMOPT_DTYPE_F32));
 }

@@ -186,6 +186,12 @@ __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, void* lds, 
                                            kStreamPolicy);
 }
 
+// The same with the default policy, for lines that other workgroups read too.
+__device__ __forceinline__ void load_lds16_cached(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0,
+                                           kLoadPolicy);
+}
+
 // Wait until at most N vector-memory loads of this wave are outstanding (loads complete in
 // issue order). The memory clobber keeps LDS reads of direct-loaded data after the wait.
 template <int N>

@@ -226,6 +226,14 @@ hipError_t launch_linear_f32_pieces(const LinearArgs& a, hipStream_t stream, boo
 // it (no workspace); *fits is false for the shapes it does not take.
 hipError_t launch_linear_oneshot_f32(const LinearArgs& a, hipStream_t stream, bool* fits);
 size_t f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int bits);
+// fp32 activations on the MFMA GEMM over exact bf16 pieces: groups and K of whole 64-wide stages;
+// *fits is false (nothing launched) for other shapes or a workspace below f32_gemm_workspace_bytes.
+hipError_t launch_linear_f32_gemm(const LinearArgs& a, hipStream_t stream, bool* fits);
+size_t f32_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group);
+// Batches of fp32 activations from this many tokens take that GEMM (given its workspace).
+int64_t f32_gemm_min_tokens(int64_t group);
+// fp32 tokens whose pieces the decode kernels take in one launch.
+int64_t f32_chunk_tokens(int64_t group);
 // Long batches in two passes: the weight dequantized into the workspace, then hipBLASLt's dense
 // GEMM. *fits is false (nothing launched) when the workspace is smaller than
 // dense_workspace_bytes, for an epilogue, or when hipBLASLt offers no algorithm for the shape.
