@@ -159,21 +159,8 @@ struct Mfma16x16<ActF16> {
 // offsets[s]; and the tile that holds that token takes its key and value from these registers
 // instead of the cache, so no workgroup waits for the store. The slot a sequence writes must not be
 // a key of another sequence in the same call (a block being filled is never shared).
-//
-// PRE: prefill, q_len query tokens per sequence. A wave holds NCB blocks of 16 B-operand columns,
-// each kTpt = 16 / GQ consecutive query tokens x the GQ heads of the KV head (block cb, column c:
-// token j0 + cb kTpt + c / GQ, head c % GQ); wave w of workgroup x takes tokens j0 = (x W + w)
-// kTpt NCB .. and every key tile up to its last token's position, so the W waves walk the same
-// key tiles together (their loads meet in the CU's L1) and each stores its own columns. A key
-// tile's K operand, slot rows and rearranged V serve all NCB blocks; each block keeps its own
-// softmax state and output. Key t enters column c's softmax iff it is a key and
-// t <= ctx - q_len + token (the reference's causal mask).
-template <class C, int HD, int GQ, int W, bool ROPE = false, bool PRE = false, int NCB = 1>
+template <class C, int HD, int GQ, int W, bool ROPE = false>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) paged_decode_kernel(const PagedDecodeArgs a) {
-  static_assert(!(ROPE && PRE), "the rotary step is a decode-step fusion");
-  static_assert(NCB == 1 || PRE, "several column blocks per wave: prefill");
-  constexpr int kNc = PRE ? 16 : GQ;  // columns of the B operand that carry queries
-  constexpr int kTpt = 16 / GQ;       // PRE: query tokens per workgroup
   constexpr int kNm = HD / 32;  // score MFMAs per tile (32 dims each)
   constexpr int kNv = HD / 16;  // P V MFMAs per tile; also V dims per lane per token
   constexpr int kVw = kNv / 2;  // 32-bit words of V per lane per token
@@ -181,36 +168,12 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
   const int wave = W > 1 ? int(threadIdx.x >> 6) : 0;
   const int col = lane & 15;
   const int kb = lane >> 4;
-  // PRE: grid (KV head, sequence, query block), the blocks latest in the prompt (the longest
-  // walks under the causal mask) dispatched first: 32 x 512-token prompts 476 -> 448 us against
-  // query blocks innermost.
-  const int64_t split = PRE ? int64_t(gridDim.z) - 1 - blockIdx.z : blockIdx.x;
-  const int64_t kvh = PRE ? blockIdx.x : blockIdx.y, s = PRE ? blockIdx.y : blockIdx.z;
+  const int64_t split = blockIdx.x, kvh = blockIdx.y, s = blockIdx.z;
   const int64_t ctx = a.context_lens[s];
-  // PRE: the wave's NCB blocks of 16 columns; block cb holds query tokens j0 + cb kTpt .. + kTpt
-  // (column col: token j0 + cb kTpt + col / GQ, head col % GQ) and the last key position each
-  // column sees (-1: none).
-  const int64_t j0 = PRE ? (split * W + wave) * kTpt * NCB : 0;
-  int64_t q_tok[NCB], q_pos[NCB];
-  bool q_ok[NCB];
-#pragma unroll
-  for (int cb = 0; cb < NCB; ++cb) {
-    q_tok[cb] = PRE ? j0 + cb * kTpt + col / GQ : 0;
-    q_ok[cb] = !PRE || q_tok[cb] < a.q_len;
-    q_pos[cb] = PRE && q_ok[cb] ? ctx - a.q_len + q_tok[cb] : -1;
-  }
-  int64_t t_begin, t_end;
-  if constexpr (PRE) {
-    const int64_t last = j0 + kTpt * NCB < a.q_len ? j0 + kTpt * NCB : a.q_len;  // tokens j0 .. last - 1
-    const int64_t lim = ctx - a.q_len + last;                         // keys t < lim
-    t_begin = 0;
-    t_end = j0 >= a.q_len ? 0 : ctx < lim ? ctx : lim;  // a wave past the prompt walks no tiles
-  } else {
-    t_begin = split * a.tiles_per_split * 16;
-    t_end = ctx < t_begin + a.tiles_per_split * 16 ? ctx : t_begin + a.tiles_per_split * 16;
-  }
+  const int64_t t_begin = split * a.tiles_per_split * 16;
+  const int64_t t_end = ctx < t_begin + a.tiles_per_split * 16 ? ctx : t_begin + a.tiles_per_split * 16;
   // The workgroup's tiles are dealt to its waves in turn: wave w takes tiles w, w + W, ...
-  auto tile_t0 = [&](int64_t j) -> int64_t { return PRE ? 16 * j : t_begin + 16 * (wave + int64_t(W) * j); };
+  auto tile_t0 = [&](int64_t j) -> int64_t { return t_begin + 16 * (wave + int64_t(W) * j); };
   const int64_t row_stride = a.kv_heads * HD;  // elements between two slots
   const uint32_t cache_bytes = uint32_t(a.num_blocks * a.block_size * row_stride * 2);
   const auto krs = make_rsrc(a.key_cache, cache_bytes);
@@ -224,7 +187,7 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
   // (q.to(k.dtype)); columns >= GQ are zero. One branch on the dtype, then independent loads.
   // ROPE: the group's rotated q heads and the rotated new key, [GQ + 1][HD] of the cache dtype.
   __shared__ __align__(16) typename C::raw rot_lds[ROPE ? (GQ + 1) * HD : 8];
-  u32x4 qf[NCB][kNm];
+  u32x4 qf[kNm];
   u32x4 knew[ROPE ? kNm : 1];     // the new key, dims 32m + 8kb .. + 8 (the K operand's order)
   uint32_t vnew[ROPE ? kVw : 1];  // the new value, dims kNv col .. + kNv (the V operand's order)
   int64_t off_new = -1;           // its position in the sequence
@@ -256,7 +219,7 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
       __syncthreads();
 #pragma unroll
       for (int m = 0; m < kNm; ++m) {
-        qf[0][m] = col < GQ ? *reinterpret_cast<const u32x4*>(rot_lds + col * HD + 32 * m + 8 * kb) : u32x4{0u, 0u, 0u, 0u};
+        qf[m] = col < GQ ? *reinterpret_cast<const u32x4*>(rot_lds + col * HD + 32 * m + 8 * kb) : u32x4{0u, 0u, 0u, 0u};
         knew[m] = *reinterpret_cast<const u32x4*>(rot_lds + GQ * HD + 32 * m + 8 * kb);
       }
       const Raw* vr = static_cast<const Raw*>(a.new_v) + s * a.ldv + kvh * HD + kNv * col;
@@ -291,59 +254,54 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
         }
       }
     } else {
+      const bool hv = col < GQ;
+      const int64_t q0 = s * a.q_seq_stride + (kvh * GQ + (hv ? col : 0)) * HD + 8 * kb;
+      float x[kNm][8];
+      // Eight consecutive dims per lane and m: one or two 16-byte loads when the rows are
+      // 16-byte aligned (a.q_vec, checked on the host), else element loads.
+      if (a.q_dtype == kDtF32) {
+        const float* q = static_cast<const float*>(a.query) + q0;
+        if (a.q_vec) {
 #pragma unroll
-      for (int cb = 0; cb < NCB; ++cb) {
-        const bool hv = PRE ? q_ok[cb] : col < GQ;
-        const int64_t q0 = PRE ? s * a.q_seq_stride + (q_ok[cb] ? q_tok[cb] : 0) * a.q_tok_stride +
-                                     (kvh * GQ + col % GQ) * a.q_head_stride + 8 * kb
-                               : s * a.q_seq_stride + (kvh * GQ + (hv ? col : 0)) * HD + 8 * kb;
-        float x[kNm][8];
-        // Eight consecutive dims per lane and m: one or two 16-byte loads when the rows are
-        // 16-byte aligned (a.q_vec, checked on the host), else element loads.
-        if (a.q_dtype == kDtF32) {
-          const float* q = static_cast<const float*>(a.query) + q0;
-          if (a.q_vec) {
+          for (int m = 0; m < kNm; ++m) {
+            const f32x4 v0 = *reinterpret_cast<const f32x4*>(q + 32 * m);
+            const f32x4 v1 = *reinterpret_cast<const f32x4*>(q + 32 * m + 4);
 #pragma unroll
-            for (int m = 0; m < kNm; ++m) {
-              const f32x4 v0 = *reinterpret_cast<const f32x4*>(q + 32 * m);
-              const f32x4 v1 = *reinterpret_cast<const f32x4*>(q + 32 * m + 4);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) x[m][e] = v0[e], x[m][e + 4] = v1[e];
-            }
-          } else {
-#pragma unroll
-            for (int m = 0; m < kNm; ++m)
-#pragma unroll
-              for (int e = 0; e < 8; ++e) x[m][e] = q[32 * m + e];
+            for (int e = 0; e < 4; ++e) x[m][e] = v0[e], x[m][e + 4] = v1[e];
           }
         } else {
-          const uint16_t* q = static_cast<const uint16_t*>(a.query) + q0;
-          const bool half = a.q_dtype == kDtF16;
-          auto cvt = [&](uint16_t h) { return half ? f16_to_f32(h) : bf16_to_f32(h); };
-          if (a.q_vec) {
 #pragma unroll
-            for (int m = 0; m < kNm; ++m) {
-              const u32x4 w = *reinterpret_cast<const u32x4*>(q + 32 * m);
-              const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+          for (int m = 0; m < kNm; ++m)
 #pragma unroll
-              for (int e = 0; e < 4; ++e)
-                x[m][2 * e] = cvt(uint16_t(ws[e])), x[m][2 * e + 1] = cvt(uint16_t(ws[e] >> 16));
-            }
-          } else {
+            for (int e = 0; e < 8; ++e) x[m][e] = q[32 * m + e];
+        }
+      } else {
+        const uint16_t* q = static_cast<const uint16_t*>(a.query) + q0;
+        const bool half = a.q_dtype == kDtF16;
+        auto cvt = [&](uint16_t h) { return half ? f16_to_f32(h) : bf16_to_f32(h); };
+        if (a.q_vec) {
 #pragma unroll
-            for (int m = 0; m < kNm; ++m)
+          for (int m = 0; m < kNm; ++m) {
+            const u32x4 w = *reinterpret_cast<const u32x4*>(q + 32 * m);
+            const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-              for (int e = 0; e < 8; ++e) x[m][e] = cvt(q[32 * m + e]);
+            for (int e = 0; e < 4; ++e)
+              x[m][2 * e] = cvt(uint16_t(ws[e])), x[m][2 * e + 1] = cvt(uint16_t(ws[e] >> 16));
           }
-        }
+        } else {
 #pragma unroll
-        for (int m = 0; m < kNm; ++m) {
-          uint32_t w[4];
+          for (int m = 0; m < kNm; ++m)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            w[e] = hv ? uint32_t(C::store(x[m][2 * e])) | (uint32_t(C::store(x[m][2 * e + 1])) << 16) : 0u;
-          qf[cb][m] = u32x4{w[0], w[1], w[2], w[3]};
+            for (int e = 0; e < 8; ++e) x[m][e] = cvt(q[32 * m + e]);
         }
+      }
+#pragma unroll
+      for (int m = 0; m < kNm; ++m) {
+        uint32_t w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          w[e] = hv ? uint32_t(C::store(x[m][2 * e])) | (uint32_t(C::store(x[m][2 * e + 1])) << 16) : 0u;
+        qf[m] = u32x4{w[0], w[1], w[2], w[3]};
       }
     }
   };
@@ -394,16 +352,11 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
   };
 
   const float neg_inf = -__int_as_float(0x7F800000);
-  float m_run[NCB], l_run[NCB];  // per column block: running max of column col (the same on
-                                 // the four lanes of a column) and this lane's share of its sum
-  f32x4 o[NCB][kNv];
+  float m_run = neg_inf, l_run = 0.0f;  // running max of column col (the same on the four lanes of
+                                        // a column) and this lane's share of its sum
+  f32x4 o[kNv];
 #pragma unroll
-  for (int cb = 0; cb < NCB; ++cb) {
-    m_run[cb] = neg_inf;
-    l_run[cb] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kNv; ++i) o[cb][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int i = 0; i < kNv; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // One tile (tokens t0 .. t0 + 15): scores, online softmax, P V, all on 64 lanes without LDS.
   auto compute = [&](const u32x4* kf_in, const uint32_t (*vf_in)[kVw], uint32_t bits, int64_t t0) {
@@ -431,57 +384,45 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
           }
       }
     }
-    // Scores of every column block against the tile's keys (the K operand shared), then each
-    // block's online softmax; the V operand is rearranged once and multiplies every block's P.
-    f32x4 acc[NCB];
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) {
-      acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < kNm; ++m) acc = Mfma16x32<C>::run(kf[m], qf[m], acc);
+    float sc[4];
 #pragma unroll
-      for (int m = 0; m < kNm; ++m) acc[cb] = Mfma16x32<C>::run(kf[m], qf[cb][m], acc[cb]);
+    for (int r = 0; r < 4; ++r) sc[r] = acc[r] * a.scale;
+    if (a.softcap > 0.0f) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sc[r] = tanhf(sc[r] / a.softcap) * a.softcap;
     }
-    u32x2 pb[NCB];
+    float tmax = neg_inf;
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) {
-      float sc[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sc[r] = acc[cb][r] * a.scale;
-      if (a.softcap > 0.0f) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sc[r] = tanhf(sc[r] / a.softcap) * a.softcap;
-      }
-      float tmax = neg_inf;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const bool key = ((bits >> (4 * kb + r)) & 1u) && (!PRE || t0 + 4 * kb + r <= q_pos[cb]);
-        sc[r] = key ? sc[r] : neg_inf;
-        tmax = fmaxf(tmax, sc[r]);
-      }
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-      const float m_new = fmaxf(m_run[cb], tmax);
-      const bool live = m_new != neg_inf;
-      const float alpha = live ? __expf(m_run[cb] - m_new) : 1.0f;
-      float p[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) p[r] = live ? __expf(sc[r] - m_new) : 0.0f;
-      l_run[cb] = alpha * l_run[cb] + ((p[0] + p[1]) + (p[2] + p[3]));
-      m_run[cb] = m_new;
-      // Rescale only when some column's max moved (alpha is exactly 1 otherwise).
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
-#pragma unroll
-        for (int i = 0; i < kNv; ++i) o[cb][i] *= alpha;
-      }
-      pb[cb] = u32x2{Mfma16x16<C>::pack(p[0], p[1]), Mfma16x16<C>::pack(p[2], p[3])};
+    for (int r = 0; r < 4; ++r) {
+      sc[r] = ((bits >> (4 * kb + r)) & 1u) ? sc[r] : neg_inf;
+      tmax = fmaxf(tmax, sc[r]);
     }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const float m_new = fmaxf(m_run, tmax);
+    const bool live = m_new != neg_inf;
+    const float alpha = live ? __expf(m_run - m_new) : 1.0f;
+    float p[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] = live ? __expf(sc[r] - m_new) : 0.0f;
+    l_run = alpha * l_run + ((p[0] + p[1]) + (p[2] + p[3]));
+    m_run = m_new;
+    // Rescale only when some column's max moved (alpha is exactly 1 otherwise).
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+#pragma unroll
+      for (int i = 0; i < kNv; ++i) o[i] *= alpha;
+    }
+    const u32x2 pb = {Mfma16x16<C>::pack(p[0], p[1]), Mfma16x16<C>::pack(p[2], p[3])};
 #pragma unroll
     for (int i = 0; i < kNv; ++i) {
       // Dim (HD/16) col + i of tokens 4kb + 0..3: half i % 2 of word i / 2 of each V piece.
       const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
       const u32x2 va = {__builtin_amdgcn_perm(vf[1][i >> 1], vf[0][i >> 1], sel),
                         __builtin_amdgcn_perm(vf[3][i >> 1], vf[2][i >> 1], sel)};
-#pragma unroll
-      for (int cb = 0; cb < NCB; ++cb) o[cb][i] = Mfma16x16<C>::run(va, pb[cb], o[cb][i]);
+      o[i] = Mfma16x16<C>::run(va, pb, o[i]);
     }
   };
 
@@ -491,13 +432,13 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
   // time. The main loop runs whole groups with unconditional loads (past the last tile they read
   // slot row 0 or nothing and are never used), so the loads keep one static order; the last
   // partial group has no refills.
-  constexpr int kDepth = PRE && NCB > 2 ? 1 : 2;  // three column blocks fit with one tile in flight
+  constexpr int kDepth = 2;
   u32x4 kf[kDepth][kNm];
   uint32_t vf[kDepth][4][kVw];
   uint32_t bits[kDepth];
   int32_t rows[kDepth];
   const int64_t n_all = t_end > t_begin ? (t_end - t_begin + 15) / 16 : 0;
-  const int64_t n_tiles = PRE ? n_all : n_all > wave ? (n_all - wave + W - 1) / W : 0;
+  const int64_t n_tiles = n_all > wave ? (n_all - wave + W - 1) / W : 0;
   if (n_tiles > 0) {
     int32_t first[kDepth];
 #pragma unroll
@@ -521,51 +462,20 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
   for (int u = 0; u < kDepth; ++u)
     if (g + u < n_tiles) compute(kf[u], vf[u], bits[u], tile_t0(g + u));
 
-  // Lane l holds column col of each column block, dims (HD/4) kb + (HD/16) r + i, unnormalized,
-  // with the wave's running max m_run and (after this sum) its running sum l_run of that column.
-#pragma unroll
-  for (int cb = 0; cb < NCB; ++cb) {
-    l_run[cb] += __shfl_xor(l_run[cb], 16, 64);
-    l_run[cb] += __shfl_xor(l_run[cb], 32, 64);
-  }
+  // Lane l holds column col, dims (HD/4) kb + (HD/16) r + i, unnormalized, with the wave's running
+  // max m_run and (after this sum) its running sum l_run of that column.
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
   const int64_t h0 = kvh * GQ;
   const int64_t d0 = (HD / 4) * kb;
-  if constexpr (PRE) {
-    const int64_t h = h0 + col % GQ;
-#pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) {
-      if (!q_ok[cb]) continue;
-      float v[4][kNv];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int i = 0; i < kNv; ++i) v[r][i] = l_run[cb] > 0.0f ? o[cb][i][r] / l_run[cb] : 0.0f;
-      const int64_t base = s * a.out_seq_stride + q_tok[cb] * a.out_tok_stride + h * a.out_head_stride + d0;
-      if (a.out_dtype == kDtF32) {
-        float* out = static_cast<float*>(a.out) + base;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int i = 0; i < kNv; ++i) out[kNv * r + i] = v[r][i];
-      } else {
-        uint16_t* out = static_cast<uint16_t*>(a.out) + base;
-        const bool half = a.out_dtype == kDtF16;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int i = 0; i < kNv; ++i) out[kNv * r + i] = half ? f32_to_f16_rne(v[r][i]) : f32_to_bf16_rne(v[r][i]);
-      }
-    }
-    return;
-  }
-  if constexpr (W == 1 && !PRE) {
+  if constexpr (W == 1) {
     if (col >= GQ) return;
     const int64_t h = h0 + col;
     float v[4][kNv];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int i = 0; i < kNv; ++i) v[r][i] = l_run[0] > 0.0f ? o[0][i][r] / l_run[0] : 0.0f;
+      for (int i = 0; i < kNv; ++i) v[r][i] = l_run > 0.0f ? o[i][r] / l_run : 0.0f;
     if (a.splits == 1) {
       const int64_t base = (s * a.num_heads + h) * HD + d0;
       if (a.out_dtype == kDtF32) {
@@ -590,24 +500,23 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int i = 0; i < kNv; ++i) part[kNv * r + i] = v[r][i];
-    if (kb == 0) a.part_lse[base] = l_run[0] > 0.0f ? m_run[0] + __logf(l_run[0]) : neg_inf;
-  } else if constexpr (!PRE) {
+    if (kb == 0) a.part_lse[base] = l_run > 0.0f ? m_run + __logf(l_run) : neg_inf;
+  } else {
     // Merge the W waves in LDS (the reference's merge_states over W parts): weights
     // exp(m_w - max m), then one (head, dim) element per thread.
-    __shared__ float m_lds[W][kNc];
-    __shared__ float l_lds[W][kNc];
-    __shared__ float o_lds[W][kNc][HD];
-    if (col < kNc) {
-      if (kb == 0) m_lds[wave][col] = m_run[0], l_lds[wave][col] = l_run[0];
+    __shared__ float m_lds[W][GQ];
+    __shared__ float l_lds[W][GQ];
+    __shared__ float o_lds[W][GQ][HD];
+    if (col < GQ) {
+      if (kb == 0) m_lds[wave][col] = m_run, l_lds[wave][col] = l_run;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int i = 0; i < kNv; ++i) o_lds[wave][col][d0 + kNv * r + i] = o[0][i][r];
+        for (int i = 0; i < kNv; ++i) o_lds[wave][col][d0 + kNv * r + i] = o[i][r];
     }
     __syncthreads();
-    for (int e = int(threadIdx.x); e < kNc * HD; e += 64 * W) {
-      const int hh = e / HD, d = e % HD;  // hh: the column (PRE: token j0 + hh / GQ, head hh % GQ)
-      if (PRE && j0 + hh / GQ >= a.q_len) continue;
+    for (int e = int(threadIdx.x); e < GQ * HD; e += 64 * W) {
+      const int hh = e / HD, d = e % HD;  // hh: the column
       float top = neg_inf;
 #pragma unroll
       for (int w = 0; w < W; ++w) top = fmaxf(top, m_lds[w][hh]);
@@ -622,10 +531,9 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
         }
       }
       const float val = lsum > 0.0f ? acc / lsum : 0.0f;
-      const int64_t h = h0 + (PRE ? hh % GQ : hh);
-      if (PRE || a.splits == 1) {
-        const int64_t i = PRE ? s * a.out_seq_stride + (j0 + hh / GQ) * a.out_tok_stride + h * a.out_head_stride + d
-                              : (s * a.num_heads + h) * HD + d;
+      const int64_t h = h0 + hh;
+      if (a.splits == 1) {
+        const int64_t i = (s * a.num_heads + h) * HD + d;
         if (a.out_dtype == kDtF32)
           static_cast<float*>(a.out)[i] = val;
         else if (a.out_dtype == kDtF16)
@@ -730,48 +638,7 @@ hipError_t launch_decode_hd(const PagedDecodeArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Blocks of 16 query columns per wave in the prefill form (two or four waves): a key tile's
-// loads, block lookups and V operand serve all of them. Measured on MI355X, 32 x 512-token
-// prompts: one block 741 us, two 520 (558 with a one-tile ring), three with a one-tile ring 476
-// (249 VGPRs), four 818 (spilling).
-constexpr int kPrefillColumnBlocks = 3;
-
-template <class C, int HD, int GQ>
-void launch_prefill_group(const PagedDecodeArgs& a, hipStream_t stream) {
-  constexpr int kTpt = 16 / GQ;
-  constexpr int kNcb = kPrefillColumnBlocks;
-  const int64_t per = int64_t(kTpt) * kNcb * a.waves;  // query tokens per workgroup
-  const dim3 grid(unsigned(a.kv_heads), unsigned(a.num_seqs), unsigned((a.q_len + per - 1) / per));
-  const int64_t per1 = int64_t(kTpt) * a.waves;
-  const dim3 grid1(unsigned(a.kv_heads), unsigned(a.num_seqs), unsigned((a.q_len + per1 - 1) / per1));
-  switch (a.waves) {
-    case 1: hipLaunchKernelGGL((paged_decode_kernel<C, HD, GQ, 1, false, true, 1>), grid1, dim3(64), 0, stream, a); break;
-    case 2: hipLaunchKernelGGL((paged_decode_kernel<C, HD, GQ, 2, false, true, kNcb>), grid, dim3(128), 0, stream, a); break;
-    default: hipLaunchKernelGGL((paged_decode_kernel<C, HD, GQ, 4, false, true, kNcb>), grid, dim3(256), 0, stream, a); break;
-  }
-}
-
-template <class C, int HD>
-hipError_t launch_prefill_hd(const PagedDecodeArgs& a, hipStream_t stream) {
-  switch (a.num_heads / a.kv_heads) {
-    case 1: launch_prefill_group<C, HD, 1>(a, stream); break;
-    case 2: launch_prefill_group<C, HD, 2>(a, stream); break;
-    case 4: launch_prefill_group<C, HD, 4>(a, stream); break;
-    case 8: launch_prefill_group<C, HD, 8>(a, stream); break;
-    case 16: launch_prefill_group<C, HD, 16>(a, stream); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
 }  // namespace
-
-hipError_t launch_paged_prefill(const PagedDecodeArgs& a, hipStream_t stream) {
-  if (a.num_seqs == 0 || a.q_len == 0) return hipSuccess;
-  if (a.cache_dtype == kDtBf16)
-    return a.head_dim == 128 ? launch_prefill_hd<ActBf16, 128>(a, stream) : launch_prefill_hd<ActBf16, 64>(a, stream);
-  return a.head_dim == 128 ? launch_prefill_hd<ActF16, 128>(a, stream) : launch_prefill_hd<ActF16, 64>(a, stream);
-}
 
 hipError_t launch_kv_write(const KvWriteArgs& a, int64_t q_len, bool decode, hipStream_t stream) {
   if (a.num_seqs == 0 || q_len == 0) return hipSuccess;
