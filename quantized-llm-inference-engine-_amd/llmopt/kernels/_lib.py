@@ -8,6 +8,8 @@ path has no host substitute.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 from pathlib import Path
@@ -24,6 +26,7 @@ __all__ = [
     "EXPORTED_SYMBOLS",
     "call",
     "library_path",
+    "load_binding",
     "load_library",
 ]
 
@@ -166,6 +169,33 @@ def load_library() -> ctypes.CDLL:
                 raise RuntimeError(f"{path} has ABI version {version}, expected {ABI_VERSION}")
             _handle = lib
     return _handle
+
+
+_binding: object | None = None
+
+
+def load_binding():  # noqa: ANN201 - the extension module
+    """Load (once) and return the native host path of the linears (``csrc/torch_binding.cpp``), with
+    the kernel library's entry points attached; raise if it has not been built."""
+    global _binding
+    if _binding is not None:
+        return _binding
+    lib = load_library()
+    with _lock:
+        if _binding is None:
+            path = Path(__file__).resolve().parent / "_llmopt_torch.so"
+            if not path.exists():
+                raise RuntimeError(f"llmopt torch binding not found at {path}; build it with "
+                                   "`python -m llmopt.kernels.build`")
+            loader = importlib.machinery.ExtensionFileLoader("_llmopt_torch", str(path))
+            spec = importlib.util.spec_from_file_location("_llmopt_torch", str(path), loader=loader)
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+            module.attach(*(ctypes.cast(getattr(lib, name), _p).value for name in (
+                "llmopt_q_linear_ex", "llmopt_q_linear_workspace_ex", "llmopt_q_linear_swiglu",
+                "llmopt_q_linear_swiglu_workspace_ex")))
+            _binding = module
+    return _binding
 
 
 def call(rc: int, what: str) -> None:

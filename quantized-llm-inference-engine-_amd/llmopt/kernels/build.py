@@ -1,4 +1,5 @@
-"""Build ``libllmopt_qlinear.so`` from ``csrc/*.hip`` with hipcc for gfx950.
+"""Build ``libllmopt_qlinear.so`` from ``csrc/*.hip`` with hipcc for gfx950, and the torch binding of
+the linears' host path, ``_llmopt_torch.so``, from ``csrc/torch_binding.cpp`` with g++.
 
 Usage: ``python -m llmopt.kernels.build`` (or :func:`build_library`). Objects go to
 ``<package>/_build/``; the library is written next to this file so it ships with the
@@ -21,6 +22,7 @@ CSRC = PACKAGE_ROOT / "csrc"
 INCLUDE = PACKAGE_ROOT.parent / "include"
 BUILD_DIR = PACKAGE_ROOT / "_build"
 LIBRARY = HERE / "libllmopt_qlinear.so"
+BINDING = HERE / "_llmopt_torch.so"  # the linears' host path (csrc/torch_binding.cpp)
 ARCH = os.environ.get("LLMOPT_OFFLOAD_ARCH", "gfx950")
 
 COMPILE_FLAGS = [
@@ -81,7 +83,9 @@ def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
 
     workers = jobs or min(len(srcs), 8)
     with ThreadPoolExecutor(max_workers=workers) as pool:
+        binding = pool.submit(build_binding, verbose)
         objs = list(pool.map(compile_one, srcs))
+        binding.result()
 
     tmp = LIBRARY.with_suffix(".so.tmp")
     link = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
@@ -97,6 +101,33 @@ def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, LIBRARY)
     return LIBRARY
+
+
+def build_binding(verbose: bool = False) -> Path:
+    """Compile ``csrc/torch_binding.cpp`` against torch into ``_llmopt_torch.so``. Always rebuilds."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    src, tmp = CSRC / "torch_binding.cpp", BINDING.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "c++", "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-isystem{root / 'include'}", f"-isystem{root / 'include/torch/csrc/api/include'}",
+           f"-isystem{sysconfig.get_paths()['include']}", f"-isystem{_rocm_include()}", str(src), "-o", str(tmp),
+           f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
+           f"-Wl,-rpath,{root / 'lib'}"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on {src.name}:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, BINDING)
+    return BINDING
+
+
+def _rocm_include() -> str:
+    return str(Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "include")
 
 
 def main() -> int:

@@ -24,12 +24,13 @@ import ctypes
 
 import torch
 
-from llmopt.kernels._lib import ALGO_AUTO, ALGO_DENSE, DTYPE_CODES, call, load_library
+from llmopt.kernels._lib import ALGO_AUTO, ALGO_DENSE, DTYPE_CODES, call, load_binding, load_library
 
 __all__ = [
     "dequantize",
     "kv_write",
     "kv_write_decode",
+    "module_linear",
     "paged_decode_attention",
     "quant_linear",
     "quant_linear_swiglu",
@@ -324,6 +325,21 @@ def quant_linear(
             "llmopt_q_linear",
         )
     return y.reshape(*lead_shape, rows)
+
+
+def module_linear(x: torch.Tensor, module, rows: int, swiglu: bool = False) -> torch.Tensor | None:  # noqa: ANN001
+    """:func:`quant_linear` (or :func:`quant_linear_swiglu`) of a module's packed buffers for the plain
+    form of a call -- contiguous tensors of the module's dtypes and shapes on one device -- with the
+    checks, allocations and the launch in native code; None for any other form, which the general
+    functions take. ``module`` holds ``qweight``, ``scales``, ``qzeros`` and ``bias`` as buffers or
+    parameters and a ``QuantLinearConfig`` as ``config``."""
+    buffers, config = module._buffers, module.config
+    bias = module._parameters.get("bias")
+    if bias is None:
+        bias = buffers.get("bias")
+    return load_binding().linear(
+        x, buffers.get("qweight"), buffers.get("scales"), buffers.get("qzeros"), bias, rows, module.in_features,
+        config.bits, config.group_size, config.symmetric, DTYPE_CODES.get(config.compute_dtype, -1), swiglu)
 
 
 ERR_WORKSPACE = -4

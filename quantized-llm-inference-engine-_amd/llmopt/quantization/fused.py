@@ -166,10 +166,12 @@ class FusedQuantLinear(_FusedBase):
         self.out_features = [p.out_features for p in parts]
 
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, ...]:
-        if x.device.type == "cuda":
+        if x.is_cuda:
             from llmopt.kernels import ops
 
-            y = ops.quant_linear(x, self.quantized_tensor(), self.bias, self.config.compute_dtype)
+            y = ops.module_linear(x, self, self.fused_out_features) if type(self) is FusedQuantLinear else None
+            if y is None:
+                y = ops.quant_linear(x, self.quantized_tensor(), self.bias, self.config.compute_dtype)
         else:
             y = self._host_product(x)
         return tuple(torch.split(y, self.out_features, dim=-1))
@@ -197,9 +199,13 @@ class QuantSwiGLU(_FusedBase):
         self.out_features = gate.out_features
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if x.device.type == "cuda":
+        if x.is_cuda:
             from llmopt.kernels import ops
 
+            if type(self) is QuantSwiGLU:
+                y = ops.module_linear(x, self, self.fused_out_features, swiglu=True)
+                if y is not None:
+                    return y
             return ops.quant_linear_swiglu(x, self.quantized_tensor(), self.bias, self.config.compute_dtype)
         y = self._host_product(x)
         blocks = y.reshape(*y.shape[:-1], self.out_features // 4, 2, 4)

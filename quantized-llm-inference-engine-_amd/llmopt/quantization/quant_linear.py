@@ -137,9 +137,13 @@ class QuantLinear(nn.Module):
         return self._cached_weight
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if x.device.type == "cuda":
+        if x.is_cuda:
             from llmopt.kernels import ops
 
+            if type(self) is QuantLinear:  # a subclass may define its own packed weight
+                y = ops.module_linear(x, self, self.out_features)
+                if y is not None:
+                    return y
             return ops.quant_linear(x, self.quantized_tensor(), self.bias, self.config.compute_dtype)
         return torch.nn.functional.linear(x, self._dequantized_weight(), self.bias)
 
