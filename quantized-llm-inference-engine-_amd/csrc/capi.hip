@@ -173,6 +173,11 @@ int run_linear(const void* x, int64_t M, int64_t K, int64_t ldx, const void* qwe
   bool fits = false;
   hipError_t err = hipSuccess;
   if (epilogue != llmopt::kEpiNone) {
+    if (K > 0 && algo == LLMOPT_ALGO_AUTO && act_dtype == LLMOPT_DTYPE_F32 &&
+        M >= llmopt::f32_gemm_min_tokens(a.group)) {
+      err = llmopt::launch_linear_f32_gemm(a, s, &fits);
+      if (fits) return hip_status(err, "fp32 linear");
+    }
     // Kernels with the fused epilogue first, unless the batch is long enough for the two-pass
     // path and the workspace holds its product and dense weight.
     const size_t temp = swiglu_temp_bytes(M, N, act_dtype);
@@ -442,8 +447,8 @@ size_t llmopt_q_linear_swiglu_workspace_ex(int64_t M, int64_t N, int64_t K, int 
                                            int act_dtype) {
   if (act_dtype != LLMOPT_DTYPE_F32) return llmopt_q_linear_swiglu_workspace(M, N, K, bits, group_size);
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  // No fp32 kernel applies the activation itself: the product into the workspace, then the
-  // combining kernel.
+  // Except for the fp32 GEMM, whose workspace is less, no fp32 kernel applies the activation itself: the
+  // product into the workspace, then the combining kernel.
   return swiglu_temp_bytes(M, N, act_dtype) + llmopt_q_linear_workspace_ex(M, N, K, bits, group_size, act_dtype);
 }
 

@@ -127,3 +127,24 @@ def test_partial_workspace_keeps_the_decode_passes():
                                  torch.cuda.current_stream().cuda_stream)
         assert rc == 0, lib.llmopt_q_last_error()
         assert float((y - full).abs().max()) <= 1e-5 * float(full.abs().max())
+
+
+@pytest.mark.parametrize("m,inter,k", [(17, 128, 128), (33, 100, 1024), (65, 516, 2048), (500, 1024, 512), (300, 14336, 256)])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_swiglu_epilogue_and_reduction(m, inter, k, with_bias):
+    # The activation in the GEMM's epilogue (no K split) and in its reduction (split): the product's fp32
+    # error, through silu(g) u, whose slopes are at most 1.1 |u| and |g|, plus a few ulp of the hardware
+    # exponential: within 2e-5 of the largest value.
+    qt, w, _ = _weight(2 * inter, k, 4, 64, True, seed=m)
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, k, generator=g).to(DEV)
+    bias = torch.randn(2 * inter, generator=g).to(DEV) if with_bias else None
+    y = ops.quant_linear_swiglu(x, qt, bias, torch.float32)
+    t = x.double() @ w.t()
+    if bias is not None:
+        t = t + bias.double()
+    blocks = t.view(m, inter // 4, 2, 4)
+    gate, up = blocks[:, :, 0].reshape(m, inter), blocks[:, :, 1].reshape(m, inter)
+    ref = gate * torch.sigmoid(gate) * up
+    assert y.shape == (m, inter)
+    assert float((y.double() - ref).abs().max()) <= 2e-5 * float(ref.abs().max())
