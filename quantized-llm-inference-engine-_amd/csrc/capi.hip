@@ -739,9 +739,10 @@ int llmopt_paged_attention_prefill(const void* query, int q_dtype, int64_t q_seq
   a.out_seq_stride = out_seq_stride;
   a.out_tok_stride = out_tok_stride;
   a.out_head_stride = out_head_stride;
-  // Waves per workgroup, each with its own 16 / group query tokens over the same key tiles.
   a.splits = 1;
-  a.waves = q_len >= 64 ? 4 : q_len >= 16 ? 2 : 1;
+  // Direct loads of the query rows: a workgroup's up to 128 tokens x 16 heads at 32-bit offsets.
+  a.q_direct = a.q_vec && q_dtype == cache_dtype && q_tok_stride < (int64_t(1) << 22) &&
+               q_head_stride < (int64_t(1) << 24);
   return hip_status(llmopt::launch_paged_prefill(a, static_cast<hipStream_t>(stream)), "prefill attention launch");
 }
 

@@ -19,12 +19,15 @@
 //     4 a + r of lane half h is key 8 a + 4 h + r of the slice. V^T comes from the row-major V tile by
 //     transposing LDS reads (ds_read_b64_tr_b16: of 16 lanes, lane 4 r + c reads dims 4 c .. of key r
 //     and lane i receives dim i of keys 0 .. 3).
-// What bounds it: the two lane-half steps around each tile -- a wave's 32 MFMAs (1024 cycles of the
-// matrix pipe) carry about as many cycles of LDS reads (each K and V fragment feeds one MFMA) and 700 of
-// softmax, so two waves per SIMD (229 registers, two workgroups of 64 KB of LDS per CU) overlap them.
+// What bounds it: long walks by issue -- per tile a wave has 32 MFMAs (1024 cycles of the matrix pipe), 48 LDS
+// reads and about 300 VALU operations with 32 exponentials among them (1700 cycles), and two waves per SIMD
+// (227 registers, two workgroups of 64 KB of LDS per CU) overlap them; short prompts by the query's and
+// output's bytes and a workgroup's start (table entry, then keys).
 // Measured (MI355X, bf16, 32 heads / 8 KV heads of 128; us against 16-row blocks per wave that read
-// their keys from L1 / L2): 32 prompts of 512 tokens 163 / 455 (423 TFLOP/s), 4 of 2048 192 / 409 (716),
-// one of 512 21.5 / 53.7, 8 chunks of 100 after 512 cached 27.7 / 72.5, 64 of 5 after 295 24.6 / 27.7.
+// their keys from L1 / L2): 32 prompts of 512 tokens 148 / 455 (467 TFLOP/s), 4 of 2048 192 / 409 (716),
+// one of 512 18.7 / 53.7, 8 chunks of 100 after 512 cached 24.4 / 72.5, 64 of 5 after 295 21.7 / 27.7. Of
+// that, against converting the query rows in registers and running all sequences' last blocks first:
+// 163 -> 148, one of 512 21.5 -> 18.7.
 //
 // K chunks are XOR-swizzled by the row's low bits (16 rows of one chunk fall on distinct banks), V
 // chunks by the key's low bits in steps of 64 bytes (the four keys of a transposing read do).
@@ -106,14 +109,13 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31, half = lane >> 5;
-  // Workgroups in the order (KV head, sequence, query block), the blocks latest in the prompt (the
-  // longest walks) first; the KV heads vary fastest, so with a multiple of eight of them every
-  // workgroup of one (sequence, KV head) runs on the same XCD and finds its keys in that L2.
+  // Workgroups in the order (KV head, query block, sequence), a sequence's last blocks (the longest walks)
+  // first: those that run together walk the keys of a few sequences, which stay in L2. The KV heads vary fastest, so with a multiple of eight of them a sequence's keys of one head are in one XCD's L2.
   const uint32_t kv_heads = uint32_t(a.kv_heads), seqs = uint32_t(a.num_seqs);
   const uint32_t blocks = gridDim.x / (kv_heads * seqs);
   const uint32_t rest = blockIdx.x / kv_heads;
-  const int64_t kvh = blockIdx.x - rest * kv_heads, s = rest % seqs;
-  const int j0 = int(blocks - 1 - rest / seqs) * kTok;
+  const int64_t kvh = blockIdx.x - rest * kv_heads, s = rest / blocks;
+  const int j0 = int(blocks - 1 - rest % blocks) * kTok;
   const int q_len = int(a.q_len);
   const int ctx = int(a.context_lens[s]);
   const int base = ctx - q_len;  // position of query token 0
@@ -127,8 +129,21 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   const int n_tiles = (t_end + kKeys - 1) / kKeys;
 
   // ---- the wave's query rows: the B operand, dims 16 m + 8 half .. of row col ----
+  // Rows of the cache dtype come in whole by direct loads into the second tile buffer (q_direct, checked on
+  // the host: 16-byte aligned rows, a workgroup's rows within 2 GiB); other dtypes and alignments convert.
   u32x4 qf[kS];
-  {
+  if (a.q_direct) {
+    const auto qrs = make_rsrc(static_cast<const uint16_t*>(a.query) + s * a.q_seq_stride + j0 * a.q_tok_stride +
+                                   kvh * GQ * a.q_head_stride, 0x7FFFFFFFu);
+#pragma unroll
+    for (int i = 0; i < 32 / kRpl; ++i) {
+      const int r = kRpl * i + lane / kCh;  // of the wave's 32
+      const int t = min(j0 + (32 * wave + r) / GQ, q_len - 1) - j0;  // rows past the chunk repeat its last token
+      load_lds16_cached(qrs, kv[1] + (32 * wave + kRpl * i) * kRowBytes,
+                        uint32_t((t * a.q_tok_stride + r % GQ * a.q_head_stride) * 2) +
+                            16 * k_chunk<HD>(r, lane % kCh), 0);
+    }
+  } else {
     const int64_t q0 = s * a.q_seq_stride + int64_t(row_ok ? tok : 0) * a.q_tok_stride +
                        (kvh * GQ + col % GQ) * a.q_head_stride + 8 * half;
     float x[kS][8];
@@ -213,9 +228,18 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   };
 
   const float neg_inf = -__int_as_float(0x7F800000);
+  // Probabilities are 2^(score c - m c), one fma and one exponential per score. c has to be positive for
+  // the maximum of the scores to be that of the exponents: a negative scale moves into the query rows, a
+  // zero one becomes too small to matter.
   const bool capped = a.softcap > 0.0f;
-  const float to_log2 = capped ? kLog2e : a.scale * kLog2e;
-  float m_run = neg_inf, l_run = 0.0f;  // running max (powers of two) of row col; this lane's share of its sum
+  const float magnitude = __builtin_fabsf(a.scale) * kLog2e;
+  const float c2 = capped ? kLog2e : magnitude > 0.0f ? magnitude : 1e-30f;
+  const uint32_t q_sign = !capped && a.scale < 0.0f ? 0x80008000u : 0u;
+  // Per row: the running maximum m_run (mc = m_run c2, 0 without keys so far), and this lane's share of
+  // the sum. (Letting the maximum lag by up to eight powers of two, so that most tiles skip the rescale, was
+  // 2 - 10 % faster and 3 - 6 % less exact: the largest probabilities are then no longer near 1, which bf16
+  // rounds least.)
+  float m_run = neg_inf, mc = 0.0f, l_run = 0.0f;
   f32x16 o[kD];
 #pragma unroll
   for (int d = 0; d < kD; ++d)
@@ -248,19 +272,17 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
         for (int v = 0; v < 16; ++v) sc[kb][v] = tanhf(sc[kb][v] * a.scale / a.softcap) * a.softcap;
     }
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) sc[kb][v] *= to_log2;
     if (mask != ~uint64_t(0) || t0 + kKeys - 1 > first_pos) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
-        const uint32_t bits = uint32_t(mask >> (32 * kb)) >> (4 * half);
-        const int room = q_pos - t0 - 32 * kb - 4 * half;  // keys past it come after this row's token
+        // Bit 8 q + r: key 8 q + 4 half + r of the block is a key at or before this row's token.
+        const int room = q_pos - t0 - 32 * kb - 4 * half;
+        const uint32_t bits = (uint32_t(mask >> (32 * kb)) >> (4 * half)) &
+                              (room >= 31 ? ~0u : room < 0 ? 0u : (2u << room) - 1u);
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int key = 8 * (v / 4) + v % 4;
-          if (!((bits >> key) & 1u) || key > room) sc[kb][v] = neg_inf;
+          const uint32_t keep = uint32_t(int32_t(bits << (31 - (8 * (v / 4) + v % 4))) >> 31);
+          sc[kb][v] = __uint_as_float((__float_as_uint(sc[kb][v]) & keep) | (__float_as_uint(neg_inf) & ~keep));
         }
       }
     }
@@ -271,16 +293,25 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       for (int v = 0; v < 16; ++v) top = fmaxf(top, sc[kb][v]);
     float t_lo, t_hi;
     halves(top, t_lo, t_hi);
-    const float m_new = fmaxf(m_run, fmaxf(t_lo, t_hi));
-    const float m_use = m_new == neg_inf ? 0.0f : m_new;  // a row without keys so far: every p is 0
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+    top = fmaxf(t_lo, t_hi);
+    if (__builtin_amdgcn_ballot_w64(top > m_run)) {
+      const float m_new = fmaxf(m_run, top);
+      const float alpha = m_run == neg_inf ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_new) * c2);
+      m_run = m_new;
+      mc = m_new == neg_inf ? 0.0f : m_new * c2;
+      l_run *= alpha;
+#pragma unroll
+      for (int d = 0; d < kD; ++d)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+    }
     u32x4 pf[2][2];
     float sum = 0.0f;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       float p[16];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) p[v] = __builtin_amdgcn_exp2f(sc[kb][v] - m_use);
+      for (int v = 0; v < 16; ++v) p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kb][v], c2, -mc));
 #pragma unroll
       for (int v = 0; v < 16; v += 4) sum += (p[v] + p[v + 1]) + (p[v + 2] + p[v + 3]);
 #pragma unroll
@@ -288,14 +319,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         pf[kb][h] = u32x4{Mfma<C>::pack(p[8 * h], p[8 * h + 1]), Mfma<C>::pack(p[8 * h + 2], p[8 * h + 3]),
                           Mfma<C>::pack(p[8 * h + 4], p[8 * h + 5]), Mfma<C>::pack(p[8 * h + 6], p[8 * h + 7])};
     }
-    l_run = alpha * l_run + sum;
-    m_run = m_new;
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
-#pragma unroll
-      for (int d = 0; d < kD; ++d)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
-    }
+    l_run += sum;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -312,6 +336,15 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   if (n_tiles > 0) {
     uint64_t mask = fetch_tile(0, fetch_entry(0), 0);
     int32_t entry = fetch_entry(kKeys);
+    if (a.q_direct) {
+      wait_vmcnt<2 * kLoads + 1>();  // the query rows: this tile's loads and the entries came after them
+#pragma unroll
+      for (int m = 0; m < kS; ++m)
+        qf[m] = *reinterpret_cast<const u32x4*>(kv[1] + (32 * wave + col) * kRowBytes +
+                                                16 * k_chunk<HD>(col, 2 * m + half));
+    }
+#pragma unroll
+    for (int m = 0; m < kS; ++m) qf[m] ^= q_sign;
     for (int i = 0; i < n_tiles; ++i) {
       const int t0 = i * kKeys, b = i & 1;
       wait_vmcnt<0>();  // this wave's rows of tile i, and the next entries
@@ -335,6 +368,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       mask = next;
     }
   }
+
+  if (n_tiles == 0) wait_vmcnt<0>();  // query rows nobody needs: they land before the LDS is used again
 
   // ---- output: row col, dims 32 d + 8 q + 4 half + r ----
   float l_lo, l_hi;

@@ -139,6 +139,7 @@ struct PagedDecodeArgs {
   // with the out_* strides.
   int64_t q_len;
   int64_t q_tok_stride, q_head_stride;
+  int q_direct;             // query rows of the cache dtype, 16-byte aligned, 128 of them within 2 GiB
   int64_t out_seq_stride, out_tok_stride, out_head_stride;
 };
 hipError_t launch_paged_decode(const PagedDecodeArgs& a, hipStream_t stream);
