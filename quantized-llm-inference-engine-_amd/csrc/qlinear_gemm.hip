@@ -559,7 +559,10 @@ __global__ void __launch_bounds__(kReduceThreads) splitk_reduce_kernel(const Lin
 // higher dequantization cost per MFMA; K splits raise it at the cost of storing and re-reading
 // fp32 partial sums that a second kernel adds up. The plan minimizes a simple time model:
 // rounds of 256 workgroups x stages per workgroup x time per stage, plus the partial-sum
-// traffic of a split, with per-stage times measured on MI355X.
+// traffic of a split, with per-stage times measured on MI355X. The heights between 128 and 256 serve
+// ragged batches over wide weights, which run in one round of fewer padded tokens (gate_up with SwiGLU, us
+// against 128- and 256-token tiles alone: 300 tokens 126 -> 94, 350 127 -> 104, 600 231 -> 187, 700 233 ->
+// 205); only the heights 64 and 128 split K, where a grid is small.
 struct GemmPlan {
   int tt = 0;      // 0: the GEMM does not take these sizes
   int splits = 1;
@@ -573,15 +576,15 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t group, int fmt) {
   if (M < 1 || N < 1 || K % kBK != 0 || group % 32 != 0) return best;
   const int gp = group % 128 == 0 ? 2 : 1;
   const int64_t units = K / kBK / gp;
-  const double stage_us[9] = {0, 0, 0.95, 0, 1.35, 0, 0, 0, 2.1};
+  const double stage_us[9] = {0, 0, 0.95, 0, 1.35, 1.54, 1.73, 1.92, 2.1};
   double best_t = 1e30;
-  for (int tt : {8, 4, 2}) {
-    if (fmt == kByte && tt == 8) continue;  // the byte-code ring does not fit the 256-token tile
+  for (int tt : {8, 7, 6, 5, 4, 2}) {
+    if (fmt == kByte && tt > 4) continue;  // the byte-code ring does not fit beyond the 128-token tile
     const int64_t tm = (M + 32 * tt - 1) / (32 * tt);
     const int64_t tn = (N + kBN - 1) / kBN;
     if (tm * tn > 0x7FFFFFFF / 8) continue;
     for (int sp = 1; sp <= 8; ++sp) {
-      if (sp > units || (tt == 8 && sp > 1)) break;  // the 256-token tile never splits
+      if (sp > units || (sp > 1 && tt != 4 && tt != 2)) break;  // only two heights split
       const int64_t wgs = tm * tn * sp;
       const int64_t rounds = (wgs + 255) / 256;
       const double stages = double((units + sp - 1) / sp * gp);
@@ -611,7 +614,7 @@ void launch_tt(const LinearArgs& a, const GemmPlan& plan, int splits, hipStream_
   // The split epilogue is a separate instantiation: its extra live values would push the
   // 256-token tile's main loop into spills. (Split results get the activation, if any, from
   // the reduction kernel.)
-  constexpr bool kCanSplit = TT < 8;
+  constexpr bool kCanSplit = TT == 4 || TT == 2;
   const int tm = int(plan.tiles_m), tn = int(plan.tiles_n);
   const bool gp2 = a.group % 128 == 0;
   if (kCanSplit && splits > 1) {
@@ -648,9 +651,14 @@ void launch_act(const LinearArgs& a, const GemmPlan& plan, int splits, hipStream
     else launch_tt<Act, 2, kByte>(a, plan, splits, stream, magic);
     return;
   }
-  if (plan.tt == 8) launch_tt<Act, 8, kNibble>(a, plan, splits, stream, magic);
-  else if (plan.tt == 4) launch_tt<Act, 4, kNibble>(a, plan, splits, stream, magic);
-  else launch_tt<Act, 2, kNibble>(a, plan, splits, stream, magic);
+  switch (plan.tt) {
+    case 8: launch_tt<Act, 8, kNibble>(a, plan, splits, stream, magic); break;
+    case 7: launch_tt<Act, 7, kNibble>(a, plan, splits, stream, magic); break;
+    case 6: launch_tt<Act, 6, kNibble>(a, plan, splits, stream, magic); break;
+    case 5: launch_tt<Act, 5, kNibble>(a, plan, splits, stream, magic); break;
+    case 4: launch_tt<Act, 4, kNibble>(a, plan, splits, stream, magic); break;
+    default: launch_tt<Act, 2, kNibble>(a, plan, splits, stream, magic); break;
+  }
 }
 
 }  // namespace
