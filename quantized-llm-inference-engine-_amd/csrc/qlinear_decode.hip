@@ -3024,10 +3024,12 @@ template <class Act, int FMT, int GS = 1>
 hipError_t launch_ks_mb(const LinearArgs& a, const KsPlan& p, uint32_t magic, hipStream_t stream) {
   if (a.M <= 16) return launch_ks_cfg<Act, 1, FMT, GS>(a, p, magic, stream);
   if (a.M <= 32) return launch_ks_cfg<Act, 2, FMT, GS>(a, p, magic, stream);
-  // Two groups per step: three token blocks (240 VGPRs); four would spill (plan_ks stops
-  // groups of 64 at 48).
-  if constexpr (GS == 1) return launch_ks_cfg<Act, 4, FMT, GS>(a, p, magic, stream);
+  // Three token blocks up to 48 tokens: a quarter of the activations, MFMAs and sums less than with four
+  // (33 / 48 tokens, us: down 24.3 / 25.7 -> 22.1 / 23.4, o 13.3 / 13.6 -> 12.1 / 12.5, 8-bit down 29.6 / 31.4
+  // -> 28.2 / 29.1).
   if (a.M <= 48) return launch_ks_cfg<Act, 3, FMT, GS>(a, p, magic, stream);
+  // Two groups per step: four token blocks would spill (plan_ks stops groups of 64 at 48).
+  if constexpr (GS == 1) return launch_ks_cfg<Act, 4, FMT, GS>(a, p, magic, stream);
   return hipErrorInvalidValue;
 }
 
