@@ -24,10 +24,11 @@
 // (227 registers, two workgroups of 64 KB of LDS per CU) overlap them; short prompts by the query's and
 // output's bytes and a workgroup's start (table entry, then keys).
 // Measured (MI355X, bf16, 32 heads / 8 KV heads of 128; us against 16-row blocks per wave that read
-// their keys from L1 / L2): 32 prompts of 512 tokens 148 / 455 (467 TFLOP/s), 4 of 2048 192 / 409 (716),
-// one of 512 18.7 / 53.7, 8 chunks of 100 after 512 cached 24.4 / 72.5, 64 of 5 after 295 21.7 / 27.7. Of
+// their keys from L1 / L2): 32 prompts of 512 tokens 132 / 455 (522 TFLOP/s), 4 of 2048 180 / 409 (762),
+// one of 512 17.6 / 53.7, 8 chunks of 100 after 512 cached 22.0 / 72.5, 64 of 5 after 295 19.2 / 27.7. Of
 // that, against converting the query rows in registers and running all sequences' last blocks first:
-// 163 -> 148, one of 512 21.5 -> 18.7.
+// 163 -> 148, one of 512 21.5 -> 18.7; the output converted in hardware pairs and slot offsets computed once
+// per key: 148 -> 132, 18.7 -> 17.6.
 //
 // K chunks are XOR-swizzled by the row's low bits (16 rows of one chunk fall on distinct banks), V
 // chunks by the key's low bits in steps of 64 bytes (the four keys of a transposing read do).
@@ -204,6 +205,13 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   const bool pow2 = (bsz & (bsz - 1)) == 0;
   const int sh = __builtin_ctz(bsz);
   auto block_of = [&](uint32_t t) -> uint32_t { return pow2 ? t >> sh : t / bsz; };
+  uint32_t k_off[kLoads], v_off_load[kLoads];  // which chunk of its row a lane brings in, per load
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int r = wave * 16 + kRpl * i + lane / kCh;
+    k_off[i] = 16 * k_chunk<HD>(r, lane % kCh);
+    v_off_load[i] = 16 * v_chunk<HD>(r, lane % kCh);
+  }
   // Lane l looks up key t0 + l: the table entry a tile ahead of the slot row it becomes.
   auto fetch_entry = [&](int t0) -> int32_t {
     const uint32_t bi = block_of(uint32_t(t0 + lane));
@@ -215,14 +223,14 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     const uint32_t t = uint32_t(t0 + lane);
     const uint32_t bi = block_of(t);
     const bool ok = int(t) < t_end && bi < ldb && entry >= 0 && uint32_t(entry) < nblk;
-    const uint32_t slot = ok ? uint32_t(entry) * bsz + (t - bi * bsz) : 0u;
+    const uint32_t slot = (ok ? uint32_t(entry) * bsz + (t - bi * bsz) : 0u) * row_stride;
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int r = wave * 16 + kRpl * i + lane / kCh;  // this lane's row of the load
-      const uint32_t row = uint32_t(__shfl(int(slot), r, 64)) * row_stride;
+      const uint32_t row = uint32_t(__shfl(int(slot), r, 64));
       uint8_t* dst = kv[b] + (wave * 16 + kRpl * i) * kRowBytes;
-      load_lds16_cached(krs, dst, row + 16 * k_chunk<HD>(r, lane % kCh), head_off);
-      load_lds16_cached(vrs, dst + kTile, row + 16 * v_chunk<HD>(r, lane % kCh), head_off);
+      load_lds16_cached(krs, dst, row + k_off[i], head_off);
+      load_lds16_cached(vrs, dst + kTile, row + v_off_load[i], head_off);
     }
     return __builtin_amdgcn_ballot_w64(ok);
   };
@@ -385,19 +393,27 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
                    reinterpret_cast<uintptr_t>(a.out) % 16 == 0;
   const bool f16 = a.out_dtype == kDtF16;
   auto narrow = [&](float v) -> uint32_t { return f16 ? f32_to_f16_rne(v) : f32_to_bf16_rne(v); };
+  // Two outputs in one word: the hardware's pair conversion for the cache dtype, the usual case.
+  const bool same = a.out_dtype == C::id;
   if (vec) {
     // Through LDS, 32 rows of the wave at a time, so that the stores are whole rows.
     wait_lgkmcnt0();
     __builtin_amdgcn_s_barrier();  // every wave is past its last tile
     uint8_t* tile = kv[0] + wave * 32 * kRowBytes;
+    auto stage_rows = [&](auto pair) {
 #pragma unroll
-    for (int d = 0; d < kD; ++d)
+      for (int d = 0; d < kD; ++d)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const u32x2 w = {narrow(value(o[d][4 * q])) | (narrow(value(o[d][4 * q + 1])) << 16),
-                         narrow(value(o[d][4 * q + 2])) | (narrow(value(o[d][4 * q + 3])) << 16)};
-        *reinterpret_cast<u32x2*>(tile + col * kRowBytes + 16 * k_chunk<HD>(col, 4 * d + q) + 8 * half) = w;
-      }
+        for (int q = 0; q < 4; ++q) {
+          const u32x2 w = {pair(value(o[d][4 * q]), value(o[d][4 * q + 1])),
+                           pair(value(o[d][4 * q + 2]), value(o[d][4 * q + 3]))};
+          *reinterpret_cast<u32x2*>(tile + col * kRowBytes + 16 * k_chunk<HD>(col, 4 * d + q) + 8 * half) = w;
+        }
+    };
+    if (same)
+      stage_rows([](float lo, float hi) { return Mfma<C>::pack(lo, hi); });
+    else
+      stage_rows([&](float lo, float hi) { return narrow(lo) | (narrow(hi) << 16); });
     wait_lgkmcnt0();  // the wave's own tile: no barrier
 #pragma unroll
     for (int i = 0; i < 32 / kRpl; ++i) {
