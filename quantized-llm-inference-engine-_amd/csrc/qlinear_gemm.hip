@@ -466,8 +466,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1
 constexpr int kReduceThreads = 64;
 // Splits whose partial sums a thread loads before adding any of them: the loads of a batch are
 // in flight together instead of one round trip per split (down at 16 tokens, 14 splits: 5.4 us
-// for the reduction with one load at a time).
-constexpr int kReduceBatch = 8;
+// for the reduction with one load at a time; 8-bit down at 3 - 32 tokens, which has 14, 0.7 - 0.9 us
+// less per call with one batch than with two of eight).
+constexpr int kReduceBatch = 16;
 
 // y[m, n] = bias[n] + sum over splits, in split order, of partials[split][m][n]: four columns
 // per thread. Deterministic: the order of the additions never depends on timing.
