@@ -52,7 +52,7 @@ def _scratch_in_loops(lines: list[str]) -> int:
 
 
 @pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not available")
-@pytest.mark.parametrize("source", ["qlinear_gemm.hip", "qlinear_decode.hip"])
+@pytest.mark.parametrize("source", ["qlinear_gemm.hip", "qlinear_gemm_f16.hip", "qlinear_decode.hip"])
 def test_no_spills_in_main_loops(tmp_path, source):
     src = build.CSRC / source
     out = tmp_path / (source + ".s")
