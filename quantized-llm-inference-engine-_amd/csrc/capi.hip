@@ -535,12 +535,21 @@ int describe_cache(llmopt::KvWriteArgs& a, void* key_cache, void* value_cache, i
 // all (two per SIMD), each with at least four 16-token tiles. Up to 8 of them (4 for groups of 16
 // query heads, whose merge buffer in LDS is larger) form one workgroup and merge in LDS; beyond
 // that the context is cut into `splits` workgroups, at most 64, which a second kernel merges.
+//
+// With heads of 128 a CU holds one workgroup of eight waves (157 registers, 187 with the rotary step),
+// so a grid of 257 - 511 of them runs in two rounds, the second nearly empty. There the split stays
+// at one round's 256 workgroups, and more than 256 pairs take workgroups of four waves, of which two share
+// a CU. Measured (MI355X, 32 / 8 heads; us against the split rounded up): 24 sequences of 320 - 640 tokens
+// 13.7 / 20.7, of 2048 - 4096 72 / 81, 9 of 1024 - 2048 18.9 / 26.5, 48 of 320 - 640 26.6 / 29.4 (28.2 / 30.1
+// with the rotary step). Past 512 pairs smaller workgroups lost (640 pairs 41.3 / 39.9, 1280 71 / 66), and
+// heads of 64 (at most 124 registers) fit two workgroups of eight waves per CU, a whole grid of up to 511.
 struct DecodePlan {
   int splits;
   int waves;
   int64_t tiles_per_split;
 };
-DecodePlan plan_decode(int64_t num_seqs, int64_t kv_heads, int64_t group, int64_t ldb, int64_t block_size) {
+DecodePlan plan_decode(int64_t num_seqs, int64_t kv_heads, int64_t head_dim, int64_t group, int64_t ldb,
+                       int64_t block_size) {
   const int64_t tiles = (ldb * block_size + 15) / 16;
   const int64_t pairs = num_seqs * kv_heads;
   const int64_t want = pairs > 0 ? (2048 + pairs - 1) / pairs : 1;
@@ -548,9 +557,11 @@ DecodePlan plan_decode(int64_t num_seqs, int64_t kv_heads, int64_t group, int64_
   if (parts > want) parts = want;
   if (parts < 1) parts = 1;
   const int wmax = group >= 16 ? 4 : 8;
+  const bool wide = head_dim == 128;
   int waves = 1;
-  while (waves < wmax && waves < parts) waves *= 2;
+  while (waves < wmax && waves < parts && !(wide && waves == 4 && pairs > 256)) waves *= 2;
   int64_t splits = (parts + waves - 1) / waves;
+  if (wide && splits > 1 && splits * waves * pairs > 2048) splits = std::max<int64_t>(1, 2048 / (waves * pairs));
   if (splits > 64) splits = 64;
   int64_t per = (tiles + splits - 1) / splits;
   if (per < 1) per = 1;
@@ -616,7 +627,7 @@ size_t llmopt_paged_attention_workspace(int64_t num_seqs, int64_t num_heads, int
                                         int64_t ldb, int64_t block_size) {
   if (num_seqs <= 0 || num_heads <= 0 || kv_heads <= 0 || head_dim <= 0 || ldb <= 0 || block_size <= 0) return 0;
   if (num_heads % kv_heads != 0) return 0;
-  const DecodePlan plan = plan_decode(num_seqs, kv_heads, num_heads / kv_heads, ldb, block_size);
+  const DecodePlan plan = plan_decode(num_seqs, kv_heads, head_dim, num_heads / kv_heads, ldb, block_size);
   if (plan.splits <= 1) return 0;
   return size_t(plan.splits) * size_t(num_seqs) * size_t(num_heads) * size_t(head_dim + 1) * sizeof(float);
 }
@@ -679,7 +690,7 @@ int prepare_paged_decode(llmopt::PagedDecodeArgs& a, const void* query, int q_dt
   a.out_dtype = q_dtype;
   const int64_t q_esize = q_dtype == LLMOPT_DTYPE_F32 ? 4 : 2;
   a.q_vec = reinterpret_cast<uintptr_t>(query) % 16 == 0 && (q_seq_stride * q_esize) % 16 == 0;
-  const DecodePlan plan = plan_decode(num_seqs, kv_heads, group, ldb, block_size);
+  const DecodePlan plan = plan_decode(num_seqs, kv_heads, head_dim, group, ldb, block_size);
   int splits = plan.splits;
   int64_t per = plan.tiles_per_split;
   const size_t need = llmopt_paged_attention_workspace(num_seqs, num_heads, kv_heads, head_dim, ldb, block_size);
