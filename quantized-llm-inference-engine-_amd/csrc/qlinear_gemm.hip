@@ -10,13 +10,15 @@ namespace {
 constexpr int kReduceThreads = 64;
 // Splits whose partial sums a thread loads before adding any of them: the loads of a batch are
 // in flight together instead of one round trip per split (down at 16 tokens, 14 splits: 5.4 us
-// for the reduction with one load at a time; 8-bit down at 3 - 32 tokens, which has 14, 0.7 - 0.9 us
-// less per call with one batch than with two of eight).
-constexpr int kReduceBatch = 16;
+// for the reduction with one load at a time). Up to eight splits, which is all the GEMM has, a batch is
+// eight: sixteen take registers that long batches miss (o at 900 tokens 58.6 us against 62.2, qkv at
+// 640 58.4 / 61.5). More, only in 8-bit K slices of the decode kernel, sixteen: 8-bit down at 3 - 32 tokens, 14
+// splits, 0.7 - 0.9 us less per call than two batches of eight.
+constexpr int kReduceBatch = 8, kReduceBatchMany = 16;
 
 // y[m, n] = bias[n] + sum over splits, in split order, of partials[split][m][n]: four columns
 // per thread. Deterministic: the order of the additions never depends on timing.
-template <class Act>
+template <class Act, int BATCH>
 __global__ void __launch_bounds__(kReduceThreads) splitk_reduce_kernel(const LinearArgs a, const float* partials, int splits) {
   using Raw = typename Act::raw;
   if (a.epilogue == kEpiSwiglu) {
@@ -29,17 +31,17 @@ __global__ void __launch_bounds__(kReduceThreads) splitk_reduce_kernel(const Lin
     const size_t plane = size_t(a.M) * a.N;
     const float* p = partials + size_t(m) * a.N + n;
     float g[4], u[4];
-    for (int s0 = 0; s0 < splits; s0 += kReduceBatch) {
-      f32x4 tg[kReduceBatch], tu[kReduceBatch];
+    for (int s0 = 0; s0 < splits; s0 += BATCH) {
+      f32x4 tg[BATCH], tu[BATCH];
 #pragma unroll
-      for (int i = 0; i < kReduceBatch; ++i) {
+      for (int i = 0; i < BATCH; ++i) {
         if (s0 + i < splits) {
           tg[i] = *reinterpret_cast<const f32x4*>(p + size_t(s0 + i) * plane);
           tu[i] = *reinterpret_cast<const f32x4*>(p + size_t(s0 + i) * plane + 4);
         }
       }
 #pragma unroll
-      for (int i = 0; i < kReduceBatch; ++i) {
+      for (int i = 0; i < BATCH; ++i) {
         if (s0 + i < splits) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -69,13 +71,13 @@ __global__ void __launch_bounds__(kReduceThreads) splitk_reduce_kernel(const Lin
   const float* p = partials + size_t(m) * a.N + n;
   float v[4] = {0.f, 0.f, 0.f, 0.f};
   if (n + 3 < a.N && a.N % 4 == 0) {
-    for (int s0 = 0; s0 < splits; s0 += kReduceBatch) {
-      f32x4 t[kReduceBatch];
+    for (int s0 = 0; s0 < splits; s0 += BATCH) {
+      f32x4 t[BATCH];
 #pragma unroll
-      for (int i = 0; i < kReduceBatch; ++i)
+      for (int i = 0; i < BATCH; ++i)
         if (s0 + i < splits) t[i] = *reinterpret_cast<const f32x4*>(p + size_t(s0 + i) * plane);
 #pragma unroll
-      for (int i = 0; i < kReduceBatch; ++i) {
+      for (int i = 0; i < BATCH; ++i) {
         if (s0 + i < splits) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] = s0 + i == 0 ? t[i][r] : v[r] + t[i][r];
@@ -147,12 +149,18 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t group, int fmt) {
 
 hipError_t launch_splitk_reduce(const LinearArgs& a, const float* partials, int splits, hipStream_t stream) {
   const int64_t threads = a.epilogue == kEpiSwiglu ? a.M * (a.N / 8) : a.M * ((a.N + 3) / 4);
-  if (a.act == kDtBf16)
-    hipLaunchKernelGGL(splitk_reduce_kernel<ActBf16>, dim3(unsigned((threads + kReduceThreads - 1) / kReduceThreads)),
-                       dim3(kReduceThreads), 0, stream, a, partials, splits);
-  else
-    hipLaunchKernelGGL(splitk_reduce_kernel<ActF16>, dim3(unsigned((threads + kReduceThreads - 1) / kReduceThreads)),
-                       dim3(kReduceThreads), 0, stream, a, partials, splits);
+  const dim3 grid(unsigned((threads + kReduceThreads - 1) / kReduceThreads)), block(kReduceThreads);
+  const bool many = splits > kReduceBatch;
+  if (a.act == kDtBf16) {
+    if (many)
+      hipLaunchKernelGGL((splitk_reduce_kernel<ActBf16, kReduceBatchMany>), grid, block, 0, stream, a, partials, splits);
+    else
+      hipLaunchKernelGGL((splitk_reduce_kernel<ActBf16, kReduceBatch>), grid, block, 0, stream, a, partials, splits);
+  } else if (many) {
+    hipLaunchKernelGGL((splitk_reduce_kernel<ActF16, kReduceBatchMany>), grid, block, 0, stream, a, partials, splits);
+  } else {
+    hipLaunchKernelGGL((splitk_reduce_kernel<ActF16, kReduceBatch>), grid, block, 0, stream, a, partials, splits);
+  }
   return hipGetLastError();
 }
 
