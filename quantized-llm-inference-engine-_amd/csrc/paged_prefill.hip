@@ -14,21 +14,24 @@
 //     row l % 32 against 16 keys per block of 32 -- keys 8 q + 4 (l / 32) + r -- so a row's softmax
 //     takes one exchange between the two lane halves;
 //   * online softmax in fp32, in powers of two; the probabilities, rounded to the cache dtype as the
-//     reference's softmax output is, are the B operand of
+//     reference's softmax output is, are summed in fp32 as rounded (v_dot2_f32: the weights of a row add up
+//     to one) and are the B operand of
 //   * O^T += V^T P^T as they lie: the MFMA sums over k, so the operands only have to agree that slot
 //     4 a + r of lane half h is key 8 a + 4 h + r of the slice. V^T comes from the row-major V tile by
 //     transposing LDS reads (ds_read_b64_tr_b16: of 16 lanes, lane 4 r + c reads dims 4 c .. of key r
 //     and lane i receives dim i of keys 0 .. 3).
 // What bounds it: long walks by issue -- per tile a wave has 32 MFMAs (1024 cycles of the matrix pipe), 48 LDS
 // reads and about 300 VALU operations with 32 exponentials among them (1700 cycles), and two waves per SIMD
-// (227 registers, two workgroups of 64 KB of LDS per CU) overlap them; short prompts by the query's and
+// (231 registers, two workgroups of 64 KB of LDS per CU) overlap them; short prompts by the query's and
 // output's bytes and a workgroup's start (table entry, then keys).
 // Measured (MI355X, bf16, 32 heads / 8 KV heads of 128; us against 16-row blocks per wave that read
-// their keys from L1 / L2): 32 prompts of 512 tokens 132 / 455 (522 TFLOP/s), 4 of 2048 180 / 409 (762),
-// one of 512 17.6 / 53.7, 8 chunks of 100 after 512 cached 22.0 / 72.5, 64 of 5 after 295 19.2 / 27.7. Of
-// that, against converting the query rows in registers and running all sequences' last blocks first:
-// 163 -> 148, one of 512 21.5 -> 18.7; the output converted in hardware pairs and slot offsets computed once
-// per key: 148 -> 132, 18.7 -> 17.6.
+// their keys from L1 / L2): 32 prompts of 512 tokens 139 / 448 (494 TFLOP/s), 4 of 2048 178 / 410 (772),
+// one of 512 18.9 / 55.4, 8 chunks of 100 after 512 cached 21.1 / 70.8, 64 of 5 after 295 18.7 / 25.1.
+// The roundings: a probability is rounded least where it is near 1, so the maximum moves in steps of 16, 16 and
+// 32 keys in the first tile, where most maxima are, and once per tile after it. 2-norm error against float64 in
+// that order, here / one step per tile and the sum of unrounded probabilities / that other kernel (steps of 16,
+// unrounded): 1.935 / 1.970 / 1.947, 1.994 / 2.022 / 2.002, 1.929 / 1.962 / 1.938, 2.181 / 2.191 / 2.179, 2.151 /
+// 2.169 / 2.149 e-3. It costs 5 % of the first figure, 2 % of the second.
 //
 // K chunks are XOR-swizzled by the row's low bits (16 rows of one chunk fall on distinct banks), V
 // chunks by the key's low bits in steps of 64 bytes (the four keys of a transposing read do).
@@ -45,6 +48,7 @@ constexpr float kLog2e = 1.44269504088896340736f;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 template <class C>
 struct Mfma;
@@ -58,6 +62,10 @@ struct Mfma<ActBf16> {
     const f32x2 v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
   }
+  __device__ static float add_pair(uint32_t pair, float sum) {  // sum + both halves, in fp32
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, 0x3F803F80u),
+                                           sum, false);
+  }
 };
 template <>
 struct Mfma<ActF16> {
@@ -68,6 +76,9 @@ struct Mfma<ActF16> {
   __device__ static uint32_t pack(float lo, float hi) {
     return uint32_t(__builtin_bit_cast(uint16_t, _Float16(lo))) |
            (uint32_t(__builtin_bit_cast(uint16_t, _Float16(hi))) << 16);
+  }
+  __device__ static float add_pair(uint32_t pair, float sum) {
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pair), __builtin_bit_cast(f16x2, 0x3C003C00u), sum, false);
   }
 };
 
@@ -111,7 +122,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31, half = lane >> 5;
   // Workgroups in the order (KV head, query block, sequence), a sequence's last blocks (the longest walks)
-  // first: those that run together walk the keys of a few sequences, which stay in L2. The KV heads vary fastest, so with a multiple of eight of them a sequence's keys of one head are in one XCD's L2.
+  // first: those that run together walk the keys of a few sequences, which stay in L2. The KV heads vary
+  // fastest, so with a multiple of eight of them a sequence's keys of one head are in one XCD's L2.
   const uint32_t kv_heads = uint32_t(a.kv_heads), seqs = uint32_t(a.num_seqs);
   const uint32_t blocks = gridDim.x / (kv_heads * seqs);
   const uint32_t rest = blockIdx.x / kv_heads;
@@ -294,51 +306,55 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         }
       }
     }
-    float top = neg_inf;
+    // Slices of 16 keys: slice i is v = 8 (i % 2) .. + 7 of block i / 2. The running maximum moves before a
+    // tile's first slice, in the first tile also before its second and third.
+    float top[4];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int i = 0; i < 4; ++i) {
+      top[i] = neg_inf;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) top = fmaxf(top, sc[kb][v]);
-    float t_lo, t_hi;
-    halves(top, t_lo, t_hi);
-    top = fmaxf(t_lo, t_hi);
-    if (__builtin_amdgcn_ballot_w64(top > m_run)) {
-      const float m_new = fmaxf(m_run, top);
-      const float alpha = m_run == neg_inf ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_new) * c2);
-      m_run = m_new;
-      mc = m_new == neg_inf ? 0.0f : m_new * c2;
-      l_run *= alpha;
-#pragma unroll
-      for (int d = 0; d < kD; ++d)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+      for (int v = 0; v < 8; ++v) top[i] = fmaxf(top[i], sc[i / 2][8 * (i % 2) + v]);
     }
-    u32x4 pf[2][2];
-    float sum = 0.0f;
+    top[2] = fmaxf(top[2], top[3]);
+    if (t0 > 0) top[0] = fmaxf(fmaxf(top[0], top[1]), top[2]);
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      float p[16];
+    for (int i = 0; i < 4; ++i) {
+      u32x4 vf[kD];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kb][v], c2, -mc));
+      for (int d = 0; d < kD; ++d) {
+        // Keys 16 i + vkey and 8 further: both have vkey's low bits, so one swizzle.
+        const uint8_t* p0 = vt + 16 * i * kRowBytes + v_off + 16 * v_chunk<HD>(vkey, 4 * d + vc);
+        const u32x2 lo = read_transposed(p0), hi = read_transposed(p0 + 8 * kRowBytes);
+        vf[d] = u32x4{lo.x, lo.y, hi.x, hi.y};
+      }
+      if (i == 0 || (t0 == 0 && i < 3)) {
+        float t_lo, t_hi;
+        halves(top[i], t_lo, t_hi);
+        const float m_new = fmaxf(m_run, fmaxf(t_lo, t_hi));
+        if (__builtin_amdgcn_ballot_w64(m_new > m_run)) {
+          const float mc_new = m_new == neg_inf ? 0.0f : m_new * c2;
+          const float alpha = m_run == neg_inf ? 0.0f : __builtin_amdgcn_exp2f(mc - mc_new);
+          m_run = m_new;
+          mc = mc_new;
+          if (i > 0 || t0 > 0) {
+            l_run *= alpha;
 #pragma unroll
-      for (int v = 0; v < 16; v += 4) sum += (p[v] + p[v + 1]) + (p[v + 2] + p[v + 3]);
+            for (int d = 0; d < kD; ++d)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        pf[kb][h] = u32x4{Mfma<C>::pack(p[8 * h], p[8 * h + 1]), Mfma<C>::pack(p[8 * h + 2], p[8 * h + 3]),
-                          Mfma<C>::pack(p[8 * h + 4], p[8 * h + 5]), Mfma<C>::pack(p[8 * h + 6], p[8 * h + 7])};
-    }
-    l_run += sum;
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int d = 0; d < kD; ++d) {
-          // Keys 32 kb + 16 h + vkey and 8 further: both have vkey's low bits, so one swizzle.
-          const uint8_t* p0 = vt + (32 * kb + 16 * h) * kRowBytes + v_off + 16 * v_chunk<HD>(vkey, 4 * d + vc);
-          const u32x2 lo = read_transposed(p0), hi = read_transposed(p0 + 8 * kRowBytes);
-          o[d] = Mfma<C>::run(u32x4{lo.x, lo.y, hi.x, hi.y}, pf[kb][h], o[d]);
+              for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+          }
         }
+      }
+      float p[8];
+#pragma unroll
+      for (int v = 0; v < 8; ++v)
+        p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i / 2][8 * (i % 2) + v], c2, -mc));
+      const u32x4 pf = {Mfma<C>::pack(p[0], p[1]), Mfma<C>::pack(p[2], p[3]), Mfma<C>::pack(p[4], p[5]),
+                        Mfma<C>::pack(p[6], p[7])};
+      l_run += Mfma<C>::add_pair(pf.w, Mfma<C>::add_pair(pf.z, Mfma<C>::add_pair(pf.y, Mfma<C>::add_pair(pf.x, 0.0f))));
+#pragma unroll
+      for (int d = 0; d < kD; ++d) o[d] = Mfma<C>::run(vf[d], pf, o[d]);
+    }
   };
 
   if (n_tiles > 0) {
