@@ -204,8 +204,8 @@ hipError_t launch_linear_decode(const LinearArgs& a, hipStream_t stream, bool* f
 hipError_t launch_linear_prefill(const LinearArgs& a, hipStream_t stream, bool* fits);
 hipError_t launch_linear_gemm(const LinearArgs& a, hipStream_t stream, bool* fits);
 // The prefill GEMM's fp16 instantiations (their own source), launched for a plan that launch_linear_gemm chose.
-void launch_gemm_f16(const LinearArgs& a, int tt, int64_t tiles_m, int64_t tiles_n, int splits, hipStream_t stream,
-                     uint32_t magic);
+hipError_t launch_gemm_f16(const LinearArgs& a, int tt, int64_t tiles_m, int64_t tiles_n, int splits,
+                           hipStream_t stream, uint32_t magic);
 // y[m, 4p + r] = silu(t[m, 8p + r]) * t[m, 8p + 4 + r] for a full fused output t [M, N]
 // (row stride ldt) in the activation dtype: the path for kernels without the fused epilogue.
 hipError_t launch_swiglu_combine(const void* t, int64_t ldt, void* y, int64_t ldy, int64_t M, int64_t N,

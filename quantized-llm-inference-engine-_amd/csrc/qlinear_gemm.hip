@@ -190,11 +190,8 @@ hipError_t launch_linear_gemm(const LinearArgs& a, hipStream_t stream, bool* fit
   const uint32_t magic =
       g == 1 ? 0u : uint32_t((uint64_t(1) << 32) / g + ((uint64_t(1) << 32) % g != 0));
   *fits = true;
-  if (a.act == kDtBf16)
-    launch_act<ActBf16>(a, plan, splits, stream, magic);
-  else
-    launch_gemm_f16(a, plan.tt, plan.tiles_m, plan.tiles_n, splits, stream, magic);
-  return hipGetLastError();
+  if (a.act == kDtBf16) return launch_act<ActBf16>(a, plan, splits, stream, magic);
+  return launch_gemm_f16(a, plan.tt, plan.tiles_m, plan.tiles_n, splits, stream, magic);
 }
 
 }  // namespace llmopt

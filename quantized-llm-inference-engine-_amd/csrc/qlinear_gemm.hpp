@@ -475,7 +475,7 @@ struct GemmPlan {
 };
 
 template <class Act, int TT, int FMT>
-void launch_tt(const LinearArgs& a, const GemmPlan& plan, int splits, hipStream_t stream, uint32_t magic) {
+hipError_t launch_tt(const LinearArgs& a, const GemmPlan& plan, int splits, hipStream_t stream, uint32_t magic) {
   float* partials = splits > 1 ? static_cast<float*>(a.workspace) : nullptr;
   const int ntiles = int(plan.tiles_m * plan.tiles_n);
   const dim3 grid(unsigned(ntiles * splits)), block(kThreads);
@@ -492,8 +492,9 @@ void launch_tt(const LinearArgs& a, const GemmPlan& plan, int splits, hipStream_
     else
       hipLaunchKernelGGL((qlinear_gemm_kernel<Act, TT, 1, kCanSplit, kEpiNone, FMT>), grid, block, 0, stream, a, tm,
                          tn, magic, splits, partials);
-    launch_splitk_reduce(a, partials, splits, stream);
-  } else if (a.epilogue == kEpiSwiglu) {
+    return launch_splitk_reduce(a, partials, splits, stream);  // reports a failed launch of the GEMM, too
+  }
+  if (a.epilogue == kEpiSwiglu) {
     if (gp2)
       hipLaunchKernelGGL((qlinear_gemm_kernel<Act, TT, 2, false, kEpiSwiglu, FMT>), grid, block, 0, stream, a, tm, tn,
                          magic, 1, partials);
@@ -508,22 +509,22 @@ void launch_tt(const LinearArgs& a, const GemmPlan& plan, int splits, hipStream_
       hipLaunchKernelGGL((qlinear_gemm_kernel<Act, TT, 1, false, kEpiNone, FMT>), grid, block, 0, stream, a, tm, tn,
                          magic, 1, partials);
   }
+  return hipGetLastError();
 }
 
 template <class Act>
-void launch_act(const LinearArgs& a, const GemmPlan& plan, int splits, hipStream_t stream, uint32_t magic) {
+hipError_t launch_act(const LinearArgs& a, const GemmPlan& plan, int splits, hipStream_t stream, uint32_t magic) {
   if (a.fmt == kByte) {  // byte codes: two code loads per tile and stage; tiles of up to 128 tokens
-    if (plan.tt == 4) launch_tt<Act, 4, kByte>(a, plan, splits, stream, magic);
-    else launch_tt<Act, 2, kByte>(a, plan, splits, stream, magic);
-    return;
+    return plan.tt == 4 ? launch_tt<Act, 4, kByte>(a, plan, splits, stream, magic)
+                        : launch_tt<Act, 2, kByte>(a, plan, splits, stream, magic);
   }
   switch (plan.tt) {
-    case 8: launch_tt<Act, 8, kNibble>(a, plan, splits, stream, magic); break;
-    case 7: launch_tt<Act, 7, kNibble>(a, plan, splits, stream, magic); break;
-    case 6: launch_tt<Act, 6, kNibble>(a, plan, splits, stream, magic); break;
-    case 5: launch_tt<Act, 5, kNibble>(a, plan, splits, stream, magic); break;
-    case 4: launch_tt<Act, 4, kNibble>(a, plan, splits, stream, magic); break;
-    default: launch_tt<Act, 2, kNibble>(a, plan, splits, stream, magic); break;
+    case 8: return launch_tt<Act, 8, kNibble>(a, plan, splits, stream, magic);
+    case 7: return launch_tt<Act, 7, kNibble>(a, plan, splits, stream, magic);
+    case 6: return launch_tt<Act, 6, kNibble>(a, plan, splits, stream, magic);
+    case 5: return launch_tt<Act, 5, kNibble>(a, plan, splits, stream, magic);
+    case 4: return launch_tt<Act, 4, kNibble>(a, plan, splits, stream, magic);
+    default: return launch_tt<Act, 2, kNibble>(a, plan, splits, stream, magic);
   }
 }
 

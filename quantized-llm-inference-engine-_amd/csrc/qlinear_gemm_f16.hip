@@ -3,14 +3,14 @@
 
 namespace llmopt {
 
-void launch_gemm_f16(const LinearArgs& a, int tt, int64_t tiles_m, int64_t tiles_n, int splits, hipStream_t stream,
-                     uint32_t magic) {
+hipError_t launch_gemm_f16(const LinearArgs& a, int tt, int64_t tiles_m, int64_t tiles_n, int splits,
+                           hipStream_t stream, uint32_t magic) {
   GemmPlan plan;
   plan.tt = tt;
   plan.splits = splits;
   plan.tiles_m = tiles_m;
   plan.tiles_n = tiles_n;
-  launch_act<ActF16>(a, plan, splits, stream, magic);
+  return launch_act<ActF16>(a, plan, splits, stream, magic);
 }
 
 }  // namespace llmopt
