@@ -10,9 +10,9 @@
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <pybind11/pybind11.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
-
-#include <exception>
 
 namespace {
 
@@ -56,73 +56,71 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     PyErr_SetString(PyExc_TypeError, "linear takes twelve arguments, after attach");
     return nullptr;
   }
-  try {
-    if (!THPVariable_CheckExact(args[0])) Py_RETURN_NONE;  // a subclass may see the general path's torch calls
-    const at::Tensor *x = tensor_of(args[0]), *qw = tensor_of(args[1]), *sc = tensor_of(args[2]);
-    const at::Tensor* zp = tensor_of(args[3]);
-    const at::Tensor* bias = tensor_of(args[4]);
-    if (!x || !qw || !sc || (!bias && args[4] != Py_None)) Py_RETURN_NONE;
-    int64_t v[7];
-    for (int i = 0; i < 7; ++i) {
-      v[i] = PyLong_AsLongLong(args[5 + i]);
-      if (v[i] == -1 && PyErr_Occurred()) {
-        PyErr_Clear();
-        Py_RETURN_NONE;
-      }
+  HANDLE_TH_ERRORS  // torch's own exception types: an allocation that fails is torch.OutOfMemoryError
+  if (!THPVariable_CheckExact(args[0])) Py_RETURN_NONE;  // a subclass may see the general path's torch calls
+  const at::Tensor *x = tensor_of(args[0]), *qw = tensor_of(args[1]), *sc = tensor_of(args[2]);
+  const at::Tensor* zp = tensor_of(args[3]);
+  const at::Tensor* bias = tensor_of(args[4]);
+  if (!x || !qw || !sc || (!bias && args[4] != Py_None)) Py_RETURN_NONE;
+  int64_t v[7];
+  for (int i = 0; i < 7; ++i) {
+    v[i] = PyLong_AsLongLong(args[5 + i]);
+    if (v[i] == -1 && PyErr_Occurred()) {
+      PyErr_Clear();
+      Py_RETURN_NONE;
     }
-    const int64_t N = v[0], K = v[1], bits = v[2], group = v[3] > 0 ? v[3] : v[1], dtype = v[5];
-    const bool symmetric = v[4] != 0, swiglu = v[6] != 0;
-    if (N < 1 || K < 1 || N > INT32_MAX || K > INT32_MAX || bits < 1 || bits > 8 || K % group != 0 || dtype < 0 ||
-        dtype > 2 || (swiglu && N % 8 != 0))
-      Py_RETURN_NONE;
-    const at::ScalarType act = dtype == 0 ? at::kFloat : dtype == 1 ? at::kHalf : at::kBFloat16;
-    const at::Device dev = x->device();
-    if (!dev.is_cuda() || x->layout() != at::kStrided || x->scalar_type() != act || x->dim() < 1 ||
-        x->size(-1) != K || !x->is_contiguous())
-      Py_RETURN_NONE;
-    const int64_t G = K / group, M = x->numel() / K;
-    if (M < 1) Py_RETURN_NONE;
-    const bool is_signed = qw->scalar_type() == at::kChar;
-    if (qw->device() != dev || !(qw->scalar_type() == at::kByte || (bits == 8 && is_signed)) || qw->dim() != 2 ||
-        qw->size(0) != N || qw->size(1) < (bits == 8 ? K : (K + 1) / 2) || !qw->is_contiguous())
-      Py_RETURN_NONE;
-    auto plain_meta = [&](const at::Tensor* t) {
-      return t && t->device() == dev && t->scalar_type() == at::kFloat && t->dim() == 2 && t->size(0) == N &&
-             t->size(1) == G && t->is_contiguous();
-    };
-    if (!plain_meta(sc) || (!symmetric && !plain_meta(zp))) Py_RETURN_NONE;
-    if (bias && (bias->device() != dev || bias->scalar_type() != act || bias->dim() != 1 || bias->size(0) != N ||
-                 !bias->is_contiguous()))
-      Py_RETURN_NONE;
+  }
+  const int64_t N = v[0], K = v[1], bits = v[2], group = v[3] > 0 ? v[3] : v[1], dtype = v[5];
+  const bool symmetric = v[4] != 0, swiglu = v[6] != 0;
+  if (N < 1 || K < 1 || N > INT32_MAX || K > INT32_MAX || bits < 1 || bits > 8 || K % group != 0 || dtype < 0 ||
+      dtype > 2 || (swiglu && N % 8 != 0))
+    Py_RETURN_NONE;
+  const at::ScalarType act = dtype == 0 ? at::kFloat : dtype == 1 ? at::kHalf : at::kBFloat16;
+  const at::Device dev = x->device();
+  if (!dev.is_cuda() || x->layout() != at::kStrided || x->scalar_type() != act || x->dim() < 1 ||
+      x->size(-1) != K || !x->is_contiguous())
+    Py_RETURN_NONE;
+  const int64_t G = K / group, M = x->numel() / K;
+  if (M < 1) Py_RETURN_NONE;
+  const bool is_signed = qw->scalar_type() == at::kChar;
+  if (qw->device() != dev || !(qw->scalar_type() == at::kByte || (bits == 8 && is_signed)) || qw->dim() != 2 ||
+      qw->size(0) != N || qw->size(1) < (bits == 8 ? K : (K + 1) / 2) || !qw->is_contiguous())
+    Py_RETURN_NONE;
+  auto plain_meta = [&](const at::Tensor* t) {
+    return t && t->device() == dev && t->scalar_type() == at::kFloat && t->dim() == 2 && t->size(0) == N &&
+           t->size(1) == G && t->is_contiguous();
+  };
+  if (!plain_meta(sc) || (!symmetric && !plain_meta(zp))) Py_RETURN_NONE;
+  if (bias && (bias->device() != dev || bias->scalar_type() != act || bias->dim() != 1 || bias->size(0) != N ||
+               !bias->is_contiguous()))
+    Py_RETURN_NONE;
 
-    const size_t ws_bytes = (swiglu ? g_api.swiglu_ws : g_api.linear_ws)(M, N, K, int(bits), int(group), int(dtype));
-    const int64_t cols = swiglu ? N / 2 : N;
-    at::Tensor y, ws;
-    {
-      const auto options = at::TensorOptions().device(dev);
-      c10::SmallVector<int64_t, 6> shape(x->sizes().begin(), x->sizes().end());
-      shape.back() = cols;
-      y = at::empty(shape, options.dtype(act));
-      if (ws_bytes) ws = at::empty({int64_t(ws_bytes)}, options.dtype(at::kByte));
-    }
-    void* stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
-    const void *xp = x->const_data_ptr(), *qp = qw->const_data_ptr();
-    const float *sp = sc->const_data_ptr<float>(), *zpp = symmetric ? nullptr : zp->const_data_ptr<float>();
-    const void* bp = bias ? bias->const_data_ptr() : nullptr;
-    void *yp = y.mutable_data_ptr(), *wp = ws_bytes ? ws.mutable_data_ptr() : nullptr;
-    int rc;
-    Py_BEGIN_ALLOW_THREADS;
+  const size_t ws_bytes = (swiglu ? g_api.swiglu_ws : g_api.linear_ws)(M, N, K, int(bits), int(group), int(dtype));
+  const int64_t cols = swiglu ? N / 2 : N;
+  at::Tensor y, ws;
+  {
+    const auto options = at::TensorOptions().device(dev);
+    c10::SmallVector<int64_t, 6> shape(x->sizes().begin(), x->sizes().end());
+    shape.back() = cols;
+    y = at::empty(shape, options.dtype(act));
+    if (ws_bytes) ws = at::empty({int64_t(ws_bytes)}, options.dtype(at::kByte));
+  }
+  void* stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+  const void *xp = x->const_data_ptr(), *qp = qw->const_data_ptr();
+  const float *sp = sc->const_data_ptr<float>(), *zpp = symmetric ? nullptr : zp->const_data_ptr<float>();
+  const void* bp = bias ? bias->const_data_ptr() : nullptr;
+  void *yp = y.mutable_data_ptr(), *wp = ws_bytes ? ws.mutable_data_ptr() : nullptr;
+  int rc;
+  {
+    pybind11::gil_scoped_release released;  // taken again also where the call throws
     rc = swiglu ? g_api.swiglu(xp, M, K, K, qp, qw->size(1), sp, zpp, bp, yp, N, cols, int(dtype), int(bits),
                                int(group), symmetric, is_signed, wp, ws_bytes, stream)
                 : g_api.linear(xp, M, K, K, qp, qw->size(1), sp, zpp, bp, yp, N, cols, int(dtype), int(bits),
                                int(group), symmetric, is_signed, wp, ws_bytes, stream, 0);
-    Py_END_ALLOW_THREADS;
-    if (rc != 0) Py_RETURN_NONE;  // the general path asks again and reports the error
-    return THPVariable_Wrap(std::move(y));
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
   }
+  if (rc != 0) Py_RETURN_NONE;  // the general path asks again and reports the error
+  return THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef methods[] = {

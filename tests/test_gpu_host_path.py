@@ -81,6 +81,26 @@ def test_other_forms_take_the_general_path():
         m(x)
 
 
+@pytest.mark.parametrize("fused", [False, True])
+def test_out_of_memory_is_torchs_own_error(fused):
+    # The output (512 MB) does not fit the share of the card that this process may take: callers catch
+    # torch.OutOfMemoryError, drop the batch and go on.
+    m = _module(4096, 256, 4, 128, False, torch.bfloat16, False)
+    m = FusedQuantLinear([m]) if fused else m
+    x = torch.zeros(65536, 256, dtype=torch.bfloat16, device=DEV)
+    small = m(x[:8])
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (128 << 20)) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            m(x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    again = m(x[:8])
+    assert all(torch.equal(a, b) for a, b in zip(again, small))
+
+
 def test_a_subclass_keeps_its_own_weight():
     class Halved(QuantLinear):
         def quantized_tensor(self):
