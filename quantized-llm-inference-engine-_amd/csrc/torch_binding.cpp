@@ -13,6 +13,7 @@
 #include <pybind11/pybind11.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 namespace {
 
@@ -133,4 +134,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_llmopt_torch", nullptr, -1, metho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__llmopt_torch(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__llmopt_torch(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}

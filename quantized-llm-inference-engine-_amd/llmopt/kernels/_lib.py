@@ -12,6 +12,7 @@ import importlib.machinery
 import importlib.util
 import os
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -24,6 +25,7 @@ __all__ = [
     "ALGO_DENSE",
     "DTYPE_CODES",
     "EXPORTED_SYMBOLS",
+    "binding_path",
     "call",
     "library_path",
     "load_binding",
@@ -172,29 +174,41 @@ def load_library() -> ctypes.CDLL:
 
 
 _binding: object | None = None
+_binding_tried = False
 
 
-def load_binding():  # noqa: ANN201 - the extension module
+def binding_path() -> Path:
+    return Path(__file__).resolve().parent / "_llmopt_torch.so"
+
+
+def load_binding():  # noqa: ANN201 - the extension module, or None
     """Load (once) and return the native host path of the linears (``csrc/torch_binding.cpp``), with
-    the kernel library's entry points attached; raise if it has not been built."""
-    global _binding
-    if _binding is not None:
+    the kernel library's entry points attached. None, with one warning, where it is not built or does not
+    load into this torch: calls then take the general path, the same kernels through ctypes."""
+    global _binding, _binding_tried
+    if _binding_tried:
         return _binding
     lib = load_library()
     with _lock:
-        if _binding is None:
-            path = Path(__file__).resolve().parent / "_llmopt_torch.so"
-            if not path.exists():
-                raise RuntimeError(f"llmopt torch binding not found at {path}; build it with "
-                                   "`python -m llmopt.kernels.build`")
-            loader = importlib.machinery.ExtensionFileLoader("_llmopt_torch", str(path))
-            spec = importlib.util.spec_from_file_location("_llmopt_torch", str(path), loader=loader)
-            module = importlib.util.module_from_spec(spec)
-            loader.exec_module(module)
-            module.attach(*(ctypes.cast(getattr(lib, name), _p).value for name in (
-                "llmopt_q_linear_ex", "llmopt_q_linear_workspace_ex", "llmopt_q_linear_swiglu",
-                "llmopt_q_linear_swiglu_workspace_ex")))
-            _binding = module
+        if not _binding_tried:
+            path = binding_path()
+            try:
+                loader = importlib.machinery.ExtensionFileLoader("_llmopt_torch", str(path))
+                spec = importlib.util.spec_from_file_location("_llmopt_torch", str(path), loader=loader)
+                module = importlib.util.module_from_spec(spec)
+                loader.exec_module(module)
+                here = torch.__version__.split("+")[0]
+                if module.torch_version != here:
+                    raise ImportError(f"built for torch {module.torch_version}, this is {here}")
+                module.attach(*(ctypes.cast(getattr(lib, name), _p).value for name in (
+                    "llmopt_q_linear_ex", "llmopt_q_linear_workspace_ex", "llmopt_q_linear_swiglu",
+                    "llmopt_q_linear_swiglu_workspace_ex")))
+                _binding = module
+            except (ImportError, OSError) as exc:
+                warnings.warn(f"the linears' native host path is not available ({exc}); calls go through ctypes, "
+                              "some 10 us longer each. Build it with `python -m llmopt.kernels.build`",
+                              RuntimeWarning, stacklevel=2)
+            _binding_tried = True
     return _binding
 
 

@@ -83,7 +83,7 @@ def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
 
     workers = jobs or min(len(srcs), 8)
     with ThreadPoolExecutor(max_workers=workers) as pool:
-        binding = pool.submit(build_binding, verbose)
+        binding = pool.submit(build_binding_if_possible, verbose)
         objs = list(pool.map(compile_one, srcs))
         binding.result()
 
@@ -124,6 +124,18 @@ def build_binding(verbose: bool = False) -> Path:
         raise RuntimeError(f"g++ failed on {src.name}:\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, BINDING)
     return BINDING
+
+
+def build_binding_if_possible(verbose: bool = False) -> Path | None:
+    """:func:`build_binding`, or None (and no binding left from an earlier build) where it does not
+    compile: the kernel library needs neither torch's headers nor a host compiler of its own, and
+    works without it."""
+    try:
+        return build_binding(verbose)
+    except (ImportError, OSError, RuntimeError) as exc:
+        BINDING.unlink(missing_ok=True)
+        print(f"the linears' native host path is left out: {exc}", file=sys.stderr, flush=True)
+        return None
 
 
 def _rocm_include() -> str:

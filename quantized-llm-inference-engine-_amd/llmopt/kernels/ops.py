@@ -331,13 +331,16 @@ def module_linear(x: torch.Tensor, module, rows: int, swiglu: bool = False) -> t
     """:func:`quant_linear` (or :func:`quant_linear_swiglu`) of a module's packed buffers for the plain
     form of a call -- contiguous tensors of the module's dtypes and shapes on one device -- with the
     checks, allocations and the launch in native code; None for any other form, which the general
-    functions take. ``module`` holds ``qweight``, ``scales``, ``qzeros`` and ``bias`` as buffers or
-    parameters and a ``QuantLinearConfig`` as ``config``."""
+    functions take, and where that path is not built. ``module`` holds ``qweight``, ``scales``,
+    ``qzeros`` and ``bias`` as buffers or parameters and a ``QuantLinearConfig`` as ``config``."""
+    binding = load_binding()
+    if binding is None:
+        return None
     buffers, config = module._buffers, module.config
     bias = module._parameters.get("bias")
     if bias is None:
         bias = buffers.get("bias")
-    return load_binding().linear(
+    return binding.linear(
         x, buffers.get("qweight"), buffers.get("scales"), buffers.get("qzeros"), bias, rows, module.in_features,
         config.bits, config.group_size, config.symmetric, DTYPE_CODES.get(config.compute_dtype, -1), swiglu)
 
