@@ -63,8 +63,7 @@ extern "C" {
 #define LLMOPT_ALGO_GENERIC 1 /* any shape and dtype; scalar dequant + fp32 dot */
 #define LLMOPT_ALGO_DECODE 2  /* MFMA skinny GEMM, M <= 64 */
 #define LLMOPT_ALGO_PREFILL 3 /* MFMA GEMM with weight tiles dequantized into LDS */
-#define LLMOPT_ALGO_DENSE 4   /* the weight dequantized into the workspace, then hipBLASLt; fp32 activations
-                                 of 65 tokens up: what AUTO runs (the same workspace is asked for) */
+#define LLMOPT_ALGO_DENSE 4   /* the weight dequantized into the workspace, then hipBLASLt */
 
 /* ABI version of the loaded library (LLMOPT_QLINEAR_ABI_VERSION). */
 int llmopt_q_abi_version(void);

@@ -205,11 +205,8 @@ int run_linear(const void* x, int64_t M, int64_t K, int64_t ldx, const void* qwe
     return hip_status(llmopt::launch_swiglu_combine(t, N, y, ldy, M, N, act_dtype, s), "swiglu launch");
   }
 
-  if (act_dtype == LLMOPT_DTYPE_F32 && M >= llmopt::f32_gemm_min_tokens(a.group) &&
-      (algo == LLMOPT_ALGO_AUTO ||
-       (algo == LLMOPT_ALGO_DENSE && dense_first(M, N, K, act_dtype, a.workspace, a.workspace_bytes)))) {
-    // fp32 activations past one decode pass: the GEMM over exact bf16 pieces, which also stands in
-    // for the dense product where that would run.
+  if (act_dtype == LLMOPT_DTYPE_F32 && algo == LLMOPT_ALGO_AUTO && M >= llmopt::f32_gemm_min_tokens(a.group)) {
+    // fp32 activations past one decode pass: the GEMM over exact bf16 pieces.
     err = llmopt::launch_linear_f32_gemm(a, s, &fits);
     if (fits) return hip_status(err, "fp32 linear");
   }

@@ -2,8 +2,8 @@
 
 This is the reference's own computation (``QuantLinear._dequantized_weight`` then ``F.linear``,
 src/llmopt/quantization/quant_linear.py:93-113), with the dense weight rebuilt in the workspace
-by every call. ``llmopt_q_linear`` takes it from 1024 tokens (65 with fp32 activations);
-``LLMOPT_ALGO_DENSE`` takes it at any size.
+by every call. ``llmopt_q_linear`` takes it from 1024 tokens (with fp32 activations from 65, for the
+shapes that the GEMM over bf16 pieces refuses); ``LLMOPT_ALGO_DENSE`` takes it at any size.
 
 * Small shapes, every storage format, each compute dtype, with and without bias: against the
   reference's sequence on the host (oracle dequantization, rounding to the compute dtype,
@@ -11,7 +11,8 @@ by every call. ``llmopt_q_linear`` takes it from 1024 tokens (65 with fp32 activ
 * The automatic choice from 1024 tokens returns exactly what ``LLMOPT_ALGO_DENSE`` returns
   (the same two launches), and stays within the bound of the fused GEMM's result.
 * fp32 activations against the product in float64: within 2e-5, the fp32 bound (the dense fp32
-  weight is exact, hipBLASLt accumulates in fp32).
+  weight is exact, hipBLASLt accumulates in fp32). The same weight described in groups of 32, which the
+  GEMM over pieces refuses, gives the bits of ``LLMOPT_ALGO_DENSE`` in groups of 64: it ran the dense product.
 * Strided rows and leading dimensions; the SwiGLU product from the two-pass path through the
   combining kernel; correct results after the plan cache has been emptied and refilled.
 """
@@ -97,10 +98,14 @@ def test_fp32_two_pass_against_float64(m):
     dqt = _to_device(qt)
     x = torch.randn(m, k, generator=torch.Generator().manual_seed(2)).to(DEV)
     bias = torch.randn(n, generator=torch.Generator().manual_seed(3)).to(DEV)
-    y = ops.quant_linear(x, dqt, bias, torch.float32)
+    y = ops.quant_linear(x, dqt, bias, torch.float32, algo=ALGO_DENSE)
     ref = x.double() @ dequantize(dqt, torch.float32).double().t() + bias.double()
     assert _rel(y, ref) <= 2e-5
-    assert torch.equal(y, ops.quant_linear(x, dqt, bias, torch.float32, algo=ALGO_DENSE))
+    assert _rel(ops.quant_linear(x, dqt, bias, torch.float32), ref) <= 2e-5  # the GEMM over pieces
+    half = QuantizedTensor(dqt.qweight, dqt.scales.repeat_interleave(2, 1), dqt.zeros.repeat_interleave(2, 1), 4, 32,
+                           True, (n, k))
+    assert torch.equal(dequantize(half, torch.float32), dequantize(dqt, torch.float32))
+    assert torch.equal(ops.quant_linear(x, half, bias, torch.float32), y)
 
 
 def test_strided_rows_and_leading_dims():
