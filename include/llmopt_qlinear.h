@@ -143,6 +143,9 @@ size_t llmopt_q_linear_dense_workspace(int64_t N, int64_t K, int act_dtype);
  * the reference dequantizes into a cached dense weight and calls F.linear.
  * x: [M, K] act_dtype with row stride ldx; y: [M, N] act_dtype with row stride ldy;
  * bias: [N] act_dtype or NULL. Accumulation is fp32. M == 0 is a no-op.
+ * LLMOPT_DTYPE_F32: batches of one pass of the decode kernels (up to 16 tokens with groups of 64, else
+ * 21) sum a group's (q - z) * x before its scale, so |x| above about 1e35 may overflow there; larger
+ * batches take the whole range.
  */
 int llmopt_q_linear(const void* x, int64_t M, int64_t K, int64_t ldx, const void* qweight,
                     int64_t ldq, const float* scales, const float* zeros, const void* bias,

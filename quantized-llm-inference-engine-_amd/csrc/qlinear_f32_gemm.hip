@@ -21,16 +21,17 @@
 // float64 (2-norm, K = 4096 / 14336): 1.7e-7 / 2.8e-7, against 1.1e-6 / 2.1e-6.
 //
 // Two kernels. split_tiles_kernel cuts x into its pieces once (truncation: each piece takes the
-// next eight significand bits, so hi + mid + lo = x exactly, nothing overflows, and an infinite or
-// NaN x is carried by hi alone) and lays them out as the GEMM's LDS images: [32-token block][64-wide
+// next eight significand bits, so hi + mid + lo = x exactly, and an infinite or NaN x is carried by hi
+// alone; rows of very large or small values are scaled first) and lays them out as the GEMM's LDS images: [32-token block][64-wide
 // k stage][piece][token][16-byte chunk, XOR-swizzled], 12 KB per block and stage, so that a stage is
 // copied to LDS by direct loads of consecutive kilobytes. f32_gemm_kernel: a workgroup of four waves
 // owns 256 output features x 32 TT tokens; each wave takes 64 features and every token, so an LDS
 // fragment read (the A operand, 32 tokens x 16 k) feeds two MFMAs and a weight fragment (the B operand,
 // one 32-bit word of packed codes per lane) is dequantized by exactly one wave and feeds 3 TT. Two
-// workgroups share a CU (72 KB of LDS and 256 registers each), which fills one's barriers, folds and
+// workgroups share a CU (72 KB of LDS and at most 224 registers each), which fills one's barriers, folds and
 // dequantization with the other's MFMAs.
 #include <algorithm>
+#include <type_traits>
 
 #include "qcommon.hpp"
 #include "qkernels.hpp"
@@ -41,6 +42,7 @@ namespace {
 constexpr int kBN = 256;        // output features per workgroup (4 waves x 64)
 constexpr int kBK = 64;         // K per stage
 constexpr int kThreads = 256;
+constexpr int kSplitThreads = 512;
 constexpr int kBuffers = 3;     // LDS stage buffers
 constexpr int kBlockBytes = 3 * 32 * kBK * 2;  // one 32-token block of one stage: three pieces
 constexpr int kMaxSplits = 16;
@@ -59,35 +61,45 @@ __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
 }
 
 // ---- x -> pieces ------------------------------------------------------------------------------------
-// Thread t: one 8-wide chunk of one token's stage. Rows past M are zero. With `sums`, also the fp32
-// sum of each (stage, token) -- read by the GEMM only for zero points that are not integers.
+// One workgroup per token; thread t takes the row's 8-wide chunks t, t + 512, ... A row whose largest finite
+// |x| lies outside 2^-64 .. 2^81 is split a second time, brought to that range by a power of two that is
+// undone on the outputs: below it the pieces' last bits fall under bf16's subnormals, above it a group's
+// unscaled sum, up to 255 |x| per product, overflows where the scaled result does not. Other rows are split
+// as they are, and so exact down to 2^-110. With `sums`, also the fp32 sum of each (stage, token) -- read by
+// the GEMM only for zero points that are not integers. Rows past M are left as they are: an MFMA's output
+// row depends on its own row only, and theirs are not stored.
+// Bound by latency at small batches: 3.0 us for 24 rows of 4096, against 2.7 without the row's range (64
+// workgroups of 256 chunks); qkv at 24 tokens 22.8 -> 23.1 us. The usual row costs its waves two ballots
+// and one exchange beside the stores; with the exact maximum found first, and held rows, it was 3.3 us.
 template <bool VEC>
-__global__ void __launch_bounds__(kThreads) split_tiles_kernel(const float* x, int64_t ldx, int64_t M, int64_t mpad,
-                                                               int ktiles, uint8_t* pieces, float* sums) {
-  const int64_t e = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  const int64_t per_row = int64_t(ktiles) * 8;
-  const int64_t m = e / per_row;
-  if (m >= mpad) return;  // mpad * per_row is a multiple of 64: whole waves leave together
-  const int c8 = int(e - m * per_row);
-  const int kt = c8 >> 3, c = c8 & 7;
-  float v[8];
-  if (m < M) {
-    const float* src = x + m * ldx + int64_t(c8) * 8;
-    if (VEC) {
-      const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
+__device__ __forceinline__ void load_chunk(const float* src, float* v) {
+  if (VEC) {
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = lo[j], v[4 + j] = hi[j];
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = src[j];
-    }
+    for (int j = 0; j < 4; ++j) v[j] = lo[j], v[4 + j] = hi[j];
   } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = 0.0f;
+    for (int j = 0; j < 8; ++j) v[j] = src[j];
   }
+}
+
+__device__ __forceinline__ uint32_t largest_finite(const float* v, uint32_t top) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t u = __float_as_uint(v[j]) & 0x7FFFFFFFu;
+    if (u < 0x7F800000u && u > top) top = u;
+  }
+  return top;
+}
+
+__device__ __forceinline__ void split_chunk(const float* in, float factor, int64_t m, int64_t mpad, int ktiles, int c8,
+                                            uint8_t* pieces, float* sums) {
+  const int kt = c8 >> 3, c = c8 & 7;
+  float v[8];
   uint32_t p[3][8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
+    v[j] = in[j] * factor;
     const uint32_t u = __float_as_uint(v[j]);
     const bool finite = (u & 0x7F800000u) != 0x7F800000u;
     // A NaN whose payload sits in the low half would truncate to infinity: keep it a NaN.
@@ -109,13 +121,62 @@ __global__ void __launch_bounds__(kThreads) split_tiles_kernel(const float* x, i
     w.w = (p[q][6] >> 16) | (p[q][7] & 0xFFFF0000u);
     *reinterpret_cast<u32x4*>(dst + q * (32 * kBK * 2)) = w;
   }
-  if (sums) {
+  if (sums) {  // the eight chunks of a stage are in eight neighbouring lanes
     float t = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     t += __shfl_xor(t, 1, 64);
     t += __shfl_xor(t, 2, 64);
     t += __shfl_xor(t, 4, 64);
     if (c == 0) sums[int64_t(kt) * mpad + m] = t;
   }
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(kSplitThreads) split_tiles_kernel(const float* x, int64_t ldx, int64_t mpad, int ktiles,
+                                                                    uint8_t* pieces, float* sums, float* undo) {
+  constexpr int kHeld = 4;  // chunks in flight per thread
+  __shared__ uint32_t seen[kSplitThreads / 64];
+  const int64_t m = blockIdx.x;
+  const int threads = int(blockDim.x), waves = threads / 64;
+  const int chunks = ktiles * 8;  // a multiple of 16: the eight lanes of a stage stay together
+  const float* row = x + m * ldx;
+  uint32_t top = 0;
+  auto split_row = [&](float factor, auto find) {
+    for (int c0 = int(threadIdx.x); c0 < chunks; c0 += kHeld * threads) {
+      float v[kHeld][8];
+#pragma unroll
+      for (int i = 0; i < kHeld; ++i)
+        if (c0 + i * threads < chunks) load_chunk<VEC>(row + int64_t(c0 + i * threads) * 8, v[i]);
+#pragma unroll
+      for (int i = 0; i < kHeld; ++i)
+        if (c0 + i * threads < chunks) {
+          if (decltype(find)::value) top = largest_finite(v[i], top);
+          split_chunk(v[i], factor, m, mpad, ktiles, c0 + i * threads, pieces, sums);
+        }
+    }
+  };
+  split_row(1.0f, std::true_type{});
+  // What the row's waves saw: anything from 2^-64 on, and anything from 2^81 on.
+  constexpr uint32_t kLow = 127 - 64, kHigh = 127 + 80;
+  const bool some = __builtin_amdgcn_ballot_w64(top >= kLow << 23) != 0;
+  const bool large = __builtin_amdgcn_ballot_w64(top >= (kHigh + 1) << 23) != 0;
+  if ((threadIdx.x & 63) == 0) seen[threadIdx.x >> 6] = (some ? 1u : 0u) | (large ? 2u : 0u);
+  __syncthreads();
+  uint32_t all = 0;
+  for (int w = 0; w < waves; ++w) all |= seen[w];
+  if (all == 1u) {  // the usual row
+    if (threadIdx.x == 0) undo[m] = 1.0f;
+    return;
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) top = max(top, uint32_t(__shfl_xor(int(top), d, 64)));
+  __syncthreads();  // the flags have been read
+  if ((threadIdx.x & 63) == 0) seen[threadIdx.x >> 6] = top;
+  __syncthreads();
+  for (int w = 0; w < waves; ++w) top = max(top, seen[w]);
+  const uint32_t e = top >> 23;  // biased exponent
+  const int shift = top == 0 ? 0 : int(e < kLow ? kLow : kHigh) - int(e);
+  if (threadIdx.x == 0) undo[m] = __uint_as_float(uint32_t(127 - shift) << 23);
+  if (shift != 0) split_row(__uint_as_float(uint32_t(127 + shift) << 23), std::false_type{});
 }
 
 // ---- codes -> exact bf16 operands -----------------------------------------------------------------
@@ -152,6 +213,7 @@ __device__ __forceinline__ u32x4 operand_bytes(uint32_t w0, uint32_t w1, float z
 struct GemmArgs {
   const uint8_t* pieces;
   const float* sums;   // [ktiles][mpad], or null: no zero points in memory
+  const float* undo;   // [mpad]: the power of two that undoes a token's scaling
   int64_t mpad;
   int tiles_m, tiles_n, splits;
   float* partials;     // splits > 1: [splits][M][N]
@@ -339,9 +401,24 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     stage(0, kt, true, PER == 1);
     stage(1, kt + 1, PER == 1, true);
   }
+  f32x4 undo[TT][4];
+  if (g.splits == 1) {  // else the reduction does it
+#pragma unroll
+    for (int j = 0; j < TT; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        undo[j][q] = *reinterpret_cast<const f32x4*>(g.undo + m0 + 32 * j + 8 * q + 4 * half);
+  }
   // Direct loads past the last stage are still in flight: they end before the LDS is released.
   wait_vmcnt<0>();
-
+  if (g.splits == 1) {
+#pragma unroll
+    for (int j = 0; j < TT; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] *= undo[j][v / 4][v % 4];
+  }
   const float* b = static_cast<const float*>(a.bias);
   if (a.epilogue == kEpiSwiglu && g.splits == 1) {
     // Fused rows 8p .. 8p + 3 are gate features 4p .. and rows 8p + 4 .. the up features (N % 8 == 0): lane
@@ -386,13 +463,15 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 
 // y = bias + the splits' partial sums, in split order; four columns per thread where they align.
 template <int V>
-__global__ void __launch_bounds__(64) f32_reduce_kernel(const LinearArgs a, const float* partials, int splits) {
+__global__ void __launch_bounds__(64) f32_reduce_kernel(const LinearArgs a, const float* partials, const float* undo,
+                                                        int splits) {
   const int64_t nv = (a.N + V - 1) / V;
   const int64_t e = int64_t(blockIdx.x) * 64 + threadIdx.x;
   if (e >= a.M * nv) return;
   const int64_t m = e / nv, n = (e - m * nv) * V;
   const size_t plane = size_t(a.M) * a.N;
   const float* p = partials + size_t(m) * a.N + n;
+  const float back = undo[m];
   typedef float vec __attribute__((ext_vector_type(V)));
   constexpr int kBatch = 8;  // planes in flight together
   vec t = {};
@@ -407,24 +486,29 @@ __global__ void __launch_bounds__(64) f32_reduce_kernel(const LinearArgs a, cons
   }
   const float* b = static_cast<const float*>(a.bias);
   float* y = static_cast<float*>(a.y) + m * a.ldy + n;
+  t *= back;
 #pragma unroll
   for (int r = 0; r < V; ++r) y[r] = b ? t[r] + b[n + r] : t[r];
 }
 
 // The same for fused gate/up columns: eight of them, four outputs, per thread (N % 8 == 0).
-__global__ void __launch_bounds__(64) f32_reduce_swiglu_kernel(const LinearArgs a, const float* partials, int splits) {
+__global__ void __launch_bounds__(64) f32_reduce_swiglu_kernel(const LinearArgs a, const float* partials,
+                                                               const float* undo, int splits) {
   const int64_t nv = a.N / 8;
   const int64_t e = int64_t(blockIdx.x) * 64 + threadIdx.x;
   if (e >= a.M * nv) return;
   const int64_t m = e / nv, n = (e - m * nv) * 8;
   const size_t plane = size_t(a.M) * a.N;
   const float* p = partials + size_t(m) * a.N + n;
+  const float back = undo[m];
   f32x4 t = *reinterpret_cast<const f32x4*>(p), u = *reinterpret_cast<const f32x4*>(p + 4);
 #pragma unroll 4
   for (int s = 1; s < splits; ++s) {
     t += *reinterpret_cast<const f32x4*>(p + size_t(s) * plane);
     u += *reinterpret_cast<const f32x4*>(p + size_t(s) * plane + 4);
   }
+  t *= back;
+  u *= back;
   const float* b = static_cast<const float*>(a.bias);
   float* y = static_cast<float*>(a.y) + m * a.ldy + n / 2;
 #pragma unroll
@@ -438,8 +522,8 @@ struct Plan {
   int splits = 1;
   int tiles_m = 0, tiles_n = 0;
   int64_t mpad = 0;
-  size_t pieces = 0, sums = 0, partials = 0;
-  size_t total() const { return pieces + sums + partials; }
+  size_t pieces = 0, sums = 0, undo = 0, partials = 0;
+  size_t total() const { return pieces + sums + undo + partials; }
 };
 
 // Tile height and K splits from a small time model, its constants measured on MI355X (sweeps of both
@@ -476,6 +560,7 @@ Plan plan(int64_t M, int64_t N, int64_t K, int64_t group) {
     best.mpad = int64_t(best.tiles_m) * 32 * best.tt;
     best.pieces = align256(size_t(best.mpad) * K * 6);
     best.sums = align256(size_t(best.mpad) * (K / kBK) * 4);
+    best.undo = align256(size_t(best.mpad) * 4);
     best.partials = best.splits > 1 ? align256(size_t(best.splits) * M * N * 4) : 0;
   }
   return best;
@@ -531,31 +616,32 @@ hipError_t launch_linear_f32_gemm(const LinearArgs& a, hipStream_t stream, bool*
   g.tiles_m = p.tiles_m;
   g.tiles_n = p.tiles_n;
   g.splits = p.splits;
-  g.partials = reinterpret_cast<float*>(ws + p.pieces + p.sums);
+  float* undo = reinterpret_cast<float*>(ws + p.pieces + p.sums);
+  g.undo = undo;
+  g.partials = reinterpret_cast<float*>(ws + p.pieces + p.sums + p.undo);
   const float* x = static_cast<const float*>(a.x);
-  const int64_t chunks = p.mpad * (a.K / 8);
-  const dim3 sgrid(unsigned((chunks + kThreads - 1) / kThreads));
+  const dim3 sgrid{unsigned(a.M)}, sblock{unsigned(std::min<int64_t>(kSplitThreads, (a.K / 8 + 63) / 64 * 64))};
   if (a.ldx % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0)
-    hipLaunchKernelGGL(split_tiles_kernel<true>, sgrid, dim3(kThreads), 0, stream, x, a.ldx, a.M, p.mpad,
-                       int(a.K / kBK), ws, sums);
+    hipLaunchKernelGGL(split_tiles_kernel<true>, sgrid, sblock, 0, stream, x, a.ldx, p.mpad,
+                       int(a.K / kBK), ws, sums, undo);
   else
-    hipLaunchKernelGGL(split_tiles_kernel<false>, sgrid, dim3(kThreads), 0, stream, x, a.ldx, a.M, p.mpad,
-                       int(a.K / kBK), ws, sums);
+    hipLaunchKernelGGL(split_tiles_kernel<false>, sgrid, sblock, 0, stream, x, a.ldx, p.mpad,
+                       int(a.K / kBK), ws, sums, undo);
   if (a.fmt == kNibble)
     p.tt == 2 ? launch_tt<2, kNibble>(a, g, stream) : launch_tt<1, kNibble>(a, g, stream);
   else
     p.tt == 2 ? launch_tt<2, kByte>(a, g, stream) : launch_tt<1, kByte>(a, g, stream);
   if (p.splits > 1 && a.epilogue == kEpiSwiglu) {
     hipLaunchKernelGGL(f32_reduce_swiglu_kernel, dim3(unsigned((a.M * (a.N / 8) + 63) / 64)), dim3(64), 0, stream, a,
-                       g.partials, p.splits);
+                       g.partials, undo, p.splits);
   } else if (p.splits > 1) {
     const bool vec = a.N % 4 == 0;
     const int64_t threads = a.M * (vec ? a.N / 4 : a.N);
     const dim3 rgrid(unsigned((threads + 63) / 64));
     if (vec)
-      hipLaunchKernelGGL(f32_reduce_kernel<4>, rgrid, dim3(64), 0, stream, a, g.partials, p.splits);
+      hipLaunchKernelGGL(f32_reduce_kernel<4>, rgrid, dim3(64), 0, stream, a, g.partials, undo, p.splits);
     else
-      hipLaunchKernelGGL(f32_reduce_kernel<1>, rgrid, dim3(64), 0, stream, a, g.partials, p.splits);
+      hipLaunchKernelGGL(f32_reduce_kernel<1>, rgrid, dim3(64), 0, stream, a, g.partials, undo, p.splits);
   }
   return hipGetLastError();
 }

@@ -99,14 +99,49 @@ def test_infinities_and_nan_match_the_dense_product():
     qt, w, _ = _weight(n, k, 4, 64, True, seed=9)
     x = torch.randn(m, k, generator=torch.Generator().manual_seed(10)).to(DEV)
     x[3, 17], x[4, 200], x[5, 0] = float("inf"), float("-inf"), float("nan")
-    x[6, 9] = 3.0e38  # finite, and rounds to infinity in bf16
+    x[6, 9] = 3.0e38  # finite, rounds to infinity in bf16, and overflows times the integer weight
     y = ops.quant_linear(x, qt, None, torch.float32)
     ref = x.double() @ w.t()
     assert torch.equal(torch.isnan(y), torch.isnan(ref))
-    assert torch.equal(torch.isposinf(y[:6]), torch.isposinf(ref[:6]))
-    assert torch.equal(torch.isneginf(y[:6]), torch.isneginf(ref[:6]))
-    rest = [0, 1, 2] + list(range(7, m))
-    assert float((y[rest].double() - ref[rest]).abs().max()) <= 1e-5 * float(ref[rest].abs().max())
+    assert torch.equal(torch.isposinf(y), torch.isposinf(ref))
+    assert torch.equal(torch.isneginf(y), torch.isneginf(ref))
+    rest = [0, 1, 2] + list(range(6, m))
+    assert bool(((y[rest].double() - ref[rest]).abs() <= 1e-5 * ref[rest].abs().amax(1, keepdim=True)).all())
+
+
+@pytest.mark.parametrize("m,n,k,bits,group,symmetric", [(40, 64, 256, 4, 64, True), (70, 300, 1024, 4, 128, False),
+                                                        (24, 6144, 4096, 4, 64, True), (65, 200, 768, 8, 768, False),
+                                                        (33, 96, 18432, 8, 128, True)])
+def test_the_whole_range_of_fp32(m, n, k, bits, group, symmetric):
+    # Rows from 2^-140 to the largest finite values, each within the error bound of its own size: nothing
+    # overflows before the scale is applied, and no bit of a small row is lost. Up to 2^-126 the bound also
+    # takes the output's own step, 2^-149.
+    qt, w, mag = _weight(n, k, bits, group, symmetric, seed=13)
+    g = torch.Generator().manual_seed(14)
+    x = torch.randn(m, k, generator=g).clamp_(-3, 3)
+    size = torch.linspace(-140, 126, m).round()
+    x = (x.double() * torch.exp2(size.double())[:, None]).float().to(DEV)
+    bound = (x.double().abs() @ mag.t()) * ((3 * group + k / group + 4) * 2.0**-23 * (1 + 2.0**-7)) + 2.0**-148
+    y, ref = ops.quant_linear(x, qt, None, torch.float32).double(), x.double() @ w.t()
+    fits = ref.abs() < 3.4e38  # else the dense product is infinite as well
+    assert bool(((y - ref).abs()[fits] <= bound[fits]).all()) and bool(torch.isinf(y[ref.abs() > 3.5e38]).all())
+
+
+def test_swiglu_of_large_and_small_rows():
+    # Each epilogue undoes the row's power of two: the one in the GEMM and the one in the reduction.
+    for m, inter, k in ((33, 100, 1024), (300, 14336, 256)):
+        qt, w, _ = _weight(2 * inter, k, 4, 64, True, seed=15)
+        x = torch.randn(m, k, generator=torch.Generator().manual_seed(16)).to(DEV)
+        y = ops.quant_linear_swiglu(x, qt, None, torch.float32)
+        x[3] *= 2.0**-100  # exact
+        x[5] *= 2.0**-70
+        z = ops.quant_linear_swiglu(x, qt, None, torch.float32)
+        keep = [i for i in range(m) if i not in (3, 5)]
+        assert torch.equal(y[keep], z[keep])
+        for r in (3, 5):  # silu(g) u is g u / 2 there
+            t = (x[r].double() @ w.t()).view(inter // 4, 2, 4)
+            ref = (t[:, 0] * t[:, 1] / 2).reshape(inter)
+            assert float((z[r].double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max()) + 2.0**-148
 
 
 def test_partial_workspace_keeps_the_decode_passes():
