@@ -83,13 +83,13 @@ __device__ __forceinline__ void load_chunk(const float* src, float* v) {
   }
 }
 
-__device__ __forceinline__ uint32_t largest_finite(const float* v, uint32_t top) {
+__device__ __forceinline__ void largest_finite(const float* v, uint32_t& top, bool& others) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const uint32_t u = __float_as_uint(v[j]) & 0x7FFFFFFFu;
+    others |= u >= 0x7F800000u;
     if (u < 0x7F800000u && u > top) top = u;
   }
-  return top;
 }
 
 __device__ __forceinline__ void split_chunk(const float* in, float factor, int64_t m, int64_t mpad, int ktiles, int c8,
@@ -140,6 +140,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_tiles_kernel(const float*
   const int chunks = ktiles * 8;  // a multiple of 16: the eight lanes of a stage stay together
   const float* row = x + m * ldx;
   uint32_t top = 0;
+  bool others = false;  // infinities or NaN
   auto split_row = [&](float factor, auto find) {
     for (int c0 = int(threadIdx.x); c0 < chunks; c0 += kHeld * threads) {
       float v[kHeld][8];
@@ -149,17 +150,18 @@ __global__ void __launch_bounds__(kSplitThreads) split_tiles_kernel(const float*
 #pragma unroll
       for (int i = 0; i < kHeld; ++i)
         if (c0 + i * threads < chunks) {
-          if (decltype(find)::value) top = largest_finite(v[i], top);
+          if (decltype(find)::value) largest_finite(v[i], top, others);
           split_chunk(v[i], factor, m, mpad, ktiles, c0 + i * threads, pieces, sums);
         }
     }
   };
   split_row(1.0f, std::true_type{});
-  // What the row's waves saw: anything from 2^-64 on, and anything from 2^81 on.
+  // What the row's waves saw: anything finite from 2^-64 on, from 2^81 on, and anything not finite.
   constexpr uint32_t kLow = 127 - 64, kHigh = 127 + 80;
   const bool some = __builtin_amdgcn_ballot_w64(top >= kLow << 23) != 0;
   const bool large = __builtin_amdgcn_ballot_w64(top >= (kHigh + 1) << 23) != 0;
-  if ((threadIdx.x & 63) == 0) seen[threadIdx.x >> 6] = (some ? 1u : 0u) | (large ? 2u : 0u);
+  const bool wild = __builtin_amdgcn_ballot_w64(others) != 0;
+  if ((threadIdx.x & 63) == 0) seen[threadIdx.x >> 6] = (some ? 1u : 0u) | (large ? 2u : 0u) | (wild ? 4u : 0u);
   __syncthreads();
   uint32_t all = 0;
   for (int w = 0; w < waves; ++w) all |= seen[w];
@@ -175,7 +177,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_tiles_kernel(const float*
   for (int w = 0; w < waves; ++w) top = max(top, seen[w]);
   const uint32_t e = top >> 23;  // biased exponent
   const int shift = top == 0 ? 0 : int(e < kLow ? kLow : kHigh) - int(e);
-  if (threadIdx.x == 0) undo[m] = __uint_as_float(uint32_t(127 - shift) << 23);
+  if (threadIdx.x == 0) undo[m] = __uint_as_float((uint32_t(127 - shift) << 23) | (all & 4u ? 0x80000000u : 0u));
   if (shift != 0) split_row(__uint_as_float(uint32_t(127 + shift) << 23), std::false_type{});
 }
 
@@ -213,7 +215,7 @@ __device__ __forceinline__ u32x4 operand_bytes(uint32_t w0, uint32_t w1, float z
 struct GemmArgs {
   const uint8_t* pieces;
   const float* sums;   // [ktiles][mpad], or null: no zero points in memory
-  const float* undo;   // [mpad]: the power of two that undoes a token's scaling
+  const float* undo;   // [mpad]: the power of two that undoes a token's scaling; negative: x holds infinities or NaN
   int64_t mpad;
   int tiles_m, tiles_n, splits;
   float* partials;     // splits > 1: [splits][M][N]
@@ -331,6 +333,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
   const f32x16 zero16 = {};
 
+  bool remainders = false;
   auto word = [](const u32x4& q, int w) { return w == 0 ? q.x : w == 1 ? q.y : w == 2 ? q.z : q.w; };
   auto stage = [&](const int u, const int kt, const bool first, const bool last) {
     wait_lgkmcnt0();       // this wave's fragment reads of stage kt - 1
@@ -372,6 +375,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
           for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_fmaf(s[i], part[i][j][v], acc[i][j][v]);
       if (ASYM && __builtin_amdgcn_ballot_w64(zr[0] != 0.0f || zr[1] != 0.0f)) {
         // A zero point that is not an integer in range: its remainder times the group's sums of x.
+        remainders = true;
 #pragma unroll 1
         for (int t = 0; t < PER; ++t) {
           const float* sum = g.sums + int64_t(kt_base + kt - t) * g.mpad + m0 + 4 * half;
@@ -390,6 +394,60 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     }
   };
 
+  // With a remainder r = z - zi, an infinite x enters a sum as (q - zi) x and as -r x, which may be NaN where
+  // (q - z) x is infinite: such a token's sum is what its infinities and NaN alone give, term by term.
+  auto redo_infinite = [&]() {
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < TT; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t m = m0 + 32 * j + 8 * q + 4 * half;
+        const f32x4 u = *reinterpret_cast<const f32x4*>(g.undo + m);  // rows past M hold anything
+#pragma unroll
+        for (int r = 0; r < 4; ++r) any |= m + r < a.M && u[r] < 0.0f;
+      }
+    if (!__builtin_amdgcn_ballot_w64(any)) return;
+#pragma unroll 1
+    for (int t = 0; t < 16 * TT; ++t) {
+      const int64_t m = m0 + 32 * (t / 16) + 8 * (t % 16 / 4) + 4 * half + t % 4;
+      const bool mine = m < a.M && g.undo[m] < 0.0f;
+      float exact[2] = {0.0f, 0.0f};
+      bool found = false;
+      if (__builtin_amdgcn_ballot_w64(mine)) {
+        const float* xm = static_cast<const float*>(a.x) + (mine ? m : 0) * a.ldx;
+#pragma unroll 1
+        for (int kt = kt_base; kt < kt_base + n_stages; ++kt) {
+          const bool here = mine && !(__builtin_fabsf(g.sums[int64_t(kt) * g.mpad + m]) < __builtin_inff());
+          if (!__builtin_amdgcn_ballot_w64(here && !(found && exact[0] != exact[0] && exact[1] != exact[1]))) continue;
+#pragma unroll 1
+          for (int k = kt * kBK; k < (kt + 1) * kBK; ++k) {
+            const float v = xm[k];
+            if (!here || __builtin_fabsf(v) < __builtin_inff()) continue;
+            found = true;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const int64_t n = min(n0 + 64 * wave + 32 * i + row, a.N - 1), gi = n * a.G + k / a.group;
+              const uint8_t* codes = a.qw + n * a.ldq;
+              const float q = FMT == kNibble     ? float((codes[k >> 1] >> (4 * (k & 1))) & 15)
+                              : a.signed_codes ? float(int8_t(codes[k]))
+                                               : float(codes[k]);
+              exact[i] += (q - a.zeros[gi]) * a.scales[gi] * v;
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < TT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          if (found && t == 16 * j + v) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[i][j][v] = exact[i];
+          }
+    }
+  };
+
   load_meta(0);
   load_codes(0, 0);
   load_codes(1, 1);
@@ -401,6 +459,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     stage(0, kt, true, PER == 1);
     stage(1, kt + 1, PER == 1, true);
   }
+  if (ASYM && remainders) redo_infinite();
   f32x4 undo[TT][4];
   if (g.splits == 1) {  // else the reduction does it
 #pragma unroll
@@ -417,7 +476,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] *= undo[j][v / 4][v % 4];
+        for (int v = 0; v < 16; ++v) acc[i][j][v] *= __builtin_fabsf(undo[j][v / 4][v % 4]);
   }
   const float* b = static_cast<const float*>(a.bias);
   if (a.epilogue == kEpiSwiglu && g.splits == 1) {
@@ -471,7 +530,7 @@ __global__ void __launch_bounds__(64) f32_reduce_kernel(const LinearArgs a, cons
   const int64_t m = e / nv, n = (e - m * nv) * V;
   const size_t plane = size_t(a.M) * a.N;
   const float* p = partials + size_t(m) * a.N + n;
-  const float back = undo[m];
+  const float back = __builtin_fabsf(undo[m]);
   typedef float vec __attribute__((ext_vector_type(V)));
   constexpr int kBatch = 8;  // planes in flight together
   vec t = {};
@@ -500,7 +559,7 @@ __global__ void __launch_bounds__(64) f32_reduce_swiglu_kernel(const LinearArgs 
   const int64_t m = e / nv, n = (e - m * nv) * 8;
   const size_t plane = size_t(a.M) * a.N;
   const float* p = partials + size_t(m) * a.N + n;
-  const float back = undo[m];
+  const float back = __builtin_fabsf(undo[m]);
   f32x4 t = *reinterpret_cast<const f32x4*>(p), u = *reinterpret_cast<const f32x4*>(p + 4);
 #pragma unroll 4
   for (int s = 1; s < splits; ++s) {

@@ -109,6 +109,28 @@ def test_infinities_and_nan_match_the_dense_product():
     assert bool(((y[rest].double() - ref[rest]).abs() <= 1e-5 * ref[rest].abs().amax(1, keepdim=True)).all())
 
 
+@pytest.mark.parametrize("zeros", ["fraction", "far"])
+@pytest.mark.parametrize("m,n,k,bits,group", [(40, 64, 256, 4, 64), (70, 300, 1024, 4, 128), (65, 257, 768, 8, 64),
+                                              (300, 512, 256, 4, 256)])
+def test_infinities_with_remainders_of_zero_points(m, n, k, bits, group, zeros):
+    # (q - z) x is infinite where (q - zi) x and (z - zi) x have opposite signs or one of them is 0 x: only a
+    # weight of exactly zero, or infinities of both signs, make a NaN. Other rows keep their values.
+    qt, w, mag = _weight(n, k, bits, group, False, seed=17, zeros=zeros)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(18)).to(DEV)
+    y0 = ops.quant_linear(x, qt, None, torch.float32)
+    _check(y0, x, w, mag, group)
+    inf = float("inf")
+    for row, at in ((3, {17: inf}), (4, {200: -inf}), (5, {0: float("nan")}), (6, {9: inf, 70: inf}),
+                    (7, {8: inf, 9: -inf}), (m - 1, {k - 1: inf, 3: 2.0e38})):
+        for c, v in at.items():
+            x[row, c] = v
+    y, ref = ops.quant_linear(x, qt, None, torch.float32), x.double() @ w.t()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    assert torch.equal(torch.isposinf(y), torch.isposinf(ref)) and torch.equal(torch.isneginf(y), torch.isneginf(ref))
+    rest = [i for i in range(m - 1) if i not in (3, 4, 5, 6, 7)]
+    assert torch.equal(y[rest], y0[rest])
+
+
 @pytest.mark.parametrize("m,n,k,bits,group,symmetric", [(40, 64, 256, 4, 64, True), (70, 300, 1024, 4, 128, False),
                                                         (24, 6144, 4096, 4, 64, True), (65, 200, 768, 8, 768, False),
                                                         (33, 96, 18432, 8, 128, True)])
