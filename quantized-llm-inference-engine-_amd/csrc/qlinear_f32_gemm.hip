@@ -577,7 +577,7 @@ __global__ void __launch_bounds__(64) f32_reduce_swiglu_kernel(const LinearArgs 
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 struct Plan {
-  int tt = 0;  // 0: not taken
+  int tt = 0;  // 0: not taken: a group or K of another size, or pieces beyond 32-bit offsets
   int splits = 1;
   int tiles_m = 0, tiles_n = 0;
   int64_t mpad = 0;
@@ -618,6 +618,7 @@ Plan plan(int64_t M, int64_t N, int64_t K, int64_t group) {
   if (best.tt) {
     best.mpad = int64_t(best.tiles_m) * 32 * best.tt;
     best.pieces = align256(size_t(best.mpad) * K * 6);
+    if (best.pieces >= size_t(1) << 31) return Plan{};
     best.sums = align256(size_t(best.mpad) * (K / kBK) * 4);
     best.undo = align256(size_t(best.mpad) * 4);
     best.partials = best.splits > 1 ? align256(size_t(best.splits) * M * N * 4) : 0;
@@ -662,7 +663,7 @@ hipError_t launch_linear_f32_gemm(const LinearArgs& a, hipStream_t stream, bool*
   if (a.ldq % 16 != 0 || reinterpret_cast<uintptr_t>(a.qw) % 16 != 0) return hipSuccess;
   if (a.N * a.ldq >= (int64_t(1) << 31) || a.N * a.G * 4 >= (int64_t(1) << 31)) return hipSuccess;
   const Plan p = plan(a.M, a.N, a.K, a.group);
-  if (p.tt == 0 || p.pieces >= (size_t(1) << 31)) return hipSuccess;
+  if (p.tt == 0) return hipSuccess;
   if (!a.workspace || a.workspace_bytes < p.total() || reinterpret_cast<uintptr_t>(a.workspace) % 256 != 0)
     return hipSuccess;
   *fits = true;

@@ -163,6 +163,18 @@ def test_fp32_takes_the_two_pass_path_from_65_tokens(lib):
     assert lib.llmopt_q_linear_workspace_ex(4096, 256, 4096, 4, 64, f32) > _dense(256, 4096, 4)
 
 
+def test_fp32_batches_beyond_the_gemm_ask_for_what_runs(lib):
+    # At K = 14336 the pieces of 24,966 tokens reach 2 GiB, which the GEMM refuses: its tiles, sums and planes
+    # are not asked for, only the dense weight's bytes or the pieces of the decode chunks.
+    f32 = _lib.DTYPE_CODES[torch.float32]
+    n, k = DOWN
+    ws = lib.llmopt_q_linear_workspace_ex
+    chunks = 3 * 4096 * 4 * 21 + ws(21, n, k, 4, 128, f32)  # sums and slices of one pass, and the rounding up
+    for m in (24961, 25000, 32768):
+        assert 6 * m * k <= ws(m, n, k, 4, 128, f32) <= 6 * m * k + chunks
+    assert ws(24960, n, k, 4, 128, f32) >= 6 * 24960 * k + 24960 * (k // 64) * 4  # taken: with the sums
+
+
 def test_wide_grids_at_33_to_64_tokens_keep_the_gemm_for_other_formats(lib):
     # 33-64 tokens over >= 1024 tiles (N >= 16384) with K < 8192 leave the split-K GEMM only
     # for the N-split decode kernel, which takes 2/4-bit codes in groups of a multiple of 128;
