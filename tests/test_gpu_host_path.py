@@ -114,20 +114,37 @@ def test_a_subclass_keeps_its_own_weight():
     assert torch.equal(m(x), y * 0.5)
 
 
-def test_side_stream_capture_and_separate_outputs():
+def test_calls_follow_the_work_before_them_on_a_side_stream():
+    # Milliseconds of products make the first input, then each call's input is the last one's output: a
+    # launch on another stream, or one that reads a buffer too early or a reused one, changes the end.
+    m = _module(4096, 4096, 4, 128, False, torch.bfloat16, False)
+    a = torch.randn(4096, 4096, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(DEV) / 64
+
+    def chain():
+        t = a
+        for _ in range(20):
+            t = t @ a
+        y, outs = t[:1] * 1.0, []
+        for i in range(20):
+            y = m(y) * (0.75 + 0.01 * i)
+            outs.append(y)
+        return torch.cat(outs)
+
+    want = chain()
+    assert bool(torch.isfinite(want.float()).all()) and len(set(want.float().norm(dim=1).tolist())) == 20
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert torch.cuda.current_stream().cuda_stream == side.cuda_stream
+        got = chain()
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(got, want)
+
+
+def test_capture_and_separate_outputs():
     m = _module(512, 4096, 4, 128, False, torch.bfloat16, False)
     x = torch.randn(1, 4096, device=DEV).to(torch.bfloat16)
     want = m(x)
-    side = torch.cuda.Stream()
-    side.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(side):
-        assert torch.cuda.current_stream().cuda_stream == side.cuda_stream
-        y = x * 1.0
-        for _ in range(20):  # each call after the work before it on this stream
-            y = (m(y)[:, :1] * 0 + 1) * x
-        z = m(y)
-    torch.cuda.current_stream().wait_stream(side)
-    assert torch.equal(z, want)
     a, b = m(x), m(x * 2)
     assert a.data_ptr() != b.data_ptr() and torch.equal(a, want)
     static = x.clone()

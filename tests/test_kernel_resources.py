@@ -2,8 +2,8 @@
 
 A change to a kernel's epilogue once raised register pressure enough that the prefill GEMM
 spilled inside its main loop, an 18x slowdown that no parity test notices. This test compiles
-the GEMM and decode sources with the library's own flags and checks that no instantiation
-touches scratch memory between its main loop's header and back edge.
+the GEMM, decode and prefill attention sources with the library's own flags and checks that no
+instantiation touches scratch memory between its main loop's header and back edge.
 """
 
 from __future__ import annotations
@@ -52,7 +52,8 @@ def _scratch_in_loops(lines: list[str]) -> int:
 
 
 @pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not available")
-@pytest.mark.parametrize("source", ["qlinear_gemm.hip", "qlinear_gemm_f16.hip", "qlinear_decode.hip"])
+@pytest.mark.parametrize("source", ["qlinear_gemm.hip", "qlinear_gemm_f16.hip", "qlinear_decode.hip",
+                                    "qlinear_f32_gemm.hip", "paged_prefill.hip"])
 def test_no_spills_in_main_loops(tmp_path, source):
     src = build.CSRC / source
     out = tmp_path / (source + ".s")
@@ -61,7 +62,7 @@ def test_no_spills_in_main_loops(tmp_path, source):
     proc = subprocess.run(cmd, capture_output=True, text=True)
     assert proc.returncode == 0, proc.stderr[-2000:]
     kernels = _kernels(out.read_text())
-    hot = {k: v for k, v in kernels.items() if "gemm_kernel" in k or "decode_" in k}
+    hot = {k: v for k, v in kernels.items() if "gemm_kernel" in k or "decode_" in k or "prefill_kernel" in k}
     assert hot, "no kernels found in the assembly"
     bad = {k: n for k, v in hot.items() if (n := _scratch_in_loops(v))}
     assert not bad, f"scratch accesses inside main loops: {bad}"
