@@ -230,7 +230,7 @@ hipError_t launch_linear_f32_pieces(const LinearArgs& a, hipStream_t stream, boo
 // it (no workspace); *fits is false for the shapes it does not take.
 hipError_t launch_linear_oneshot_f32(const LinearArgs& a, hipStream_t stream, bool* fits);
 size_t f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int bits);
-// fp32 activations on the MFMA GEMM over exact bf16 pieces: groups and K of whole 64-wide stages;
+// fp32 activations on the MFMA GEMM over exact bf16 pieces: groups of whole 64-wide stages, K of whole pairs of them;
 // *fits is false (nothing launched) for other shapes or a workspace below f32_gemm_workspace_bytes.
 hipError_t launch_linear_f32_gemm(const LinearArgs& a, hipStream_t stream, bool* fits);
 size_t f32_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group);

@@ -61,16 +61,18 @@ __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
 }
 
 // ---- x -> pieces ------------------------------------------------------------------------------------
-// One workgroup per token; thread t takes the row's 8-wide chunks t, t + 512, ... A row whose largest finite
-// |x| lies outside 2^-64 .. 2^81 is split a second time, brought to that range by a power of two that is
-// undone on the outputs: below it the pieces' last bits fall under bf16's subnormals, above it a group's
-// unscaled sum, up to 255 |x| per product, overflows where the scaled result does not. Other rows are split
-// as they are, and so exact down to 2^-110. With `sums`, also the fp32 sum of each (stage, token) -- read by
-// the GEMM only for zero points that are not integers. Rows past M are left as they are: an MFMA's output
-// row depends on its own row only, and theirs are not stored.
-// Bound by latency at small batches: 3.0 us for 24 rows of 4096, against 2.7 without the row's range (64
-// workgroups of 256 chunks); qkv at 24 tokens 22.8 -> 23.1 us. The usual row costs its waves two ballots
-// and one exchange beside the stores; with the exact maximum found first, and held rows, it was 3.3 us.
+// A row's 8-wide chunks go to the threads in turn; with `parts` (a power of two) > 1 workgroups per row, each
+// sees all of them and splits every parts-th round (small batches: few rows for many CUs). A row whose
+// largest finite |x| lies outside 2^-64 .. 2^81 is split a second time, brought to that range by a power of
+// two that is undone on the outputs: below it the pieces' last bits fall under bf16's subnormals, above it a
+// group's unscaled sum, up to 255 |x| per product, overflows where the scaled result does not. Other rows
+// are split as they are, and so exact down to 2^-110. With `sums`, also the fp32 sum of each (stage, token)
+// -- read by the GEMM only for zero points that are not integers. Rows past M are left as they are: an
+// MFMA's output row depends on its own row only, and theirs are not stored.
+// Bound by latency at small batches: 3.0 us for 24 rows of 4096, 5.1 for 32 of 14336, against 2.7 and 5.1
+// without the row's range; qkv at 24 tokens 22.7 -> 23.2 us, MLP at 32 77.9 -> 79.8. The usual row costs two
+// ballots and one exchange beside the stores. One workgroup of 512 threads per row, whatever its length: 3.2
+// and about 6.5 us; the row held and its exact maximum found first: 3.3 at 24 rows of 4096.
 template <bool VEC>
 __device__ __forceinline__ void load_chunk(const float* src, float* v) {
   if (VEC) {
@@ -80,15 +82,6 @@ __device__ __forceinline__ void load_chunk(const float* src, float* v) {
   } else {
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = src[j];
-  }
-}
-
-__device__ __forceinline__ void largest_finite(const float* v, uint32_t& top, bool& others) {
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const uint32_t u = __float_as_uint(v[j]) & 0x7FFFFFFFu;
-    others |= u >= 0x7F800000u;
-    if (u < 0x7F800000u && u > top) top = u;
   }
 }
 
@@ -132,17 +125,18 @@ __device__ __forceinline__ void split_chunk(const float* in, float factor, int64
 
 template <bool VEC>
 __global__ void __launch_bounds__(kSplitThreads) split_tiles_kernel(const float* x, int64_t ldx, int64_t mpad, int ktiles,
-                                                                    uint8_t* pieces, float* sums, float* undo) {
+                                                                    int parts, uint8_t* pieces, float* sums,
+                                                                    float* undo) {
   constexpr int kHeld = 4;  // chunks in flight per thread
   __shared__ uint32_t seen[kSplitThreads / 64];
   const int64_t m = blockIdx.x;
+  const int part = blockIdx.y;
   const int threads = int(blockDim.x), waves = threads / 64;
   const int chunks = ktiles * 8;  // a multiple of 16: the eight lanes of a stage stay together
   const float* row = x + m * ldx;
-  uint32_t top = 0;
-  bool others = false;  // infinities or NaN
+  float most = 0.0f;  // the largest |x| but NaN
   auto split_row = [&](float factor, auto find) {
-    for (int c0 = int(threadIdx.x); c0 < chunks; c0 += kHeld * threads) {
+    for (int c0 = int(threadIdx.x), round = 0; c0 < chunks; c0 += kHeld * threads, round += kHeld) {
       float v[kHeld][8];
 #pragma unroll
       for (int i = 0; i < kHeld; ++i)
@@ -150,34 +144,57 @@ __global__ void __launch_bounds__(kSplitThreads) split_tiles_kernel(const float*
 #pragma unroll
       for (int i = 0; i < kHeld; ++i)
         if (c0 + i * threads < chunks) {
-          if (decltype(find)::value) largest_finite(v[i], top, others);
-          split_chunk(v[i], factor, m, mpad, ktiles, c0 + i * threads, pieces, sums);
+          if (decltype(find)::value) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) most = fmaxf(most, __builtin_fabsf(v[i][j]));
+          }
+          if (((round + i) & (parts - 1)) == part)
+            split_chunk(v[i], factor, m, mpad, ktiles, c0 + i * threads, pieces, sums);
         }
     }
   };
   split_row(1.0f, std::true_type{});
-  // What the row's waves saw: anything finite from 2^-64 on, from 2^81 on, and anything not finite.
+  // What the row's waves saw: anything from 2^-64 on, and anything from 2^81 on.
   constexpr uint32_t kLow = 127 - 64, kHigh = 127 + 80;
-  const bool some = __builtin_amdgcn_ballot_w64(top >= kLow << 23) != 0;
-  const bool large = __builtin_amdgcn_ballot_w64(top >= (kHigh + 1) << 23) != 0;
-  const bool wild = __builtin_amdgcn_ballot_w64(others) != 0;
-  if ((threadIdx.x & 63) == 0) seen[threadIdx.x >> 6] = (some ? 1u : 0u) | (large ? 2u : 0u) | (wild ? 4u : 0u);
+  const bool some = __builtin_amdgcn_ballot_w64(most >= __uint_as_float(kLow << 23)) != 0;
+  const bool large = __builtin_amdgcn_ballot_w64(most >= __uint_as_float((kHigh + 1) << 23)) != 0;
+  if ((threadIdx.x & 63) == 0) seen[threadIdx.x >> 6] = (some ? 1u : 0u) | (large ? 2u : 0u);
   __syncthreads();
   uint32_t all = 0;
   for (int w = 0; w < waves; ++w) all |= seen[w];
+  const bool first = threadIdx.x == 0 && part == 0;
   if (all == 1u) {  // the usual row
-    if (threadIdx.x == 0) undo[m] = 1.0f;
+    if (first) undo[m] = 1.0f;
     return;
   }
+  // The largest finite |x|, and whether there is anything else.
+  uint32_t top = 0, others = 0;
+  for (int c8 = int(threadIdx.x); c8 < chunks; c8 += threads) {
+    float v[8];
+    load_chunk<VEC>(row + int64_t(c8) * 8, v);
 #pragma unroll
-  for (int d = 1; d < 64; d *= 2) top = max(top, uint32_t(__shfl_xor(int(top), d, 64)));
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t u = __float_as_uint(v[j]) & 0x7FFFFFFFu;
+      if (u >= 0x7F800000u)
+        others = 0x80000000u;
+      else if (u > top)
+        top = u;
+    }
+  }
+  top |= others;  // in the sign bit
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) {
+    const uint32_t t = uint32_t(__shfl_xor(int(top), d, 64));
+    top = max(top & 0x7FFFFFFFu, t & 0x7FFFFFFFu) | ((top | t) & 0x80000000u);
+  }
   __syncthreads();  // the flags have been read
   if ((threadIdx.x & 63) == 0) seen[threadIdx.x >> 6] = top;
   __syncthreads();
-  for (int w = 0; w < waves; ++w) top = max(top, seen[w]);
-  const uint32_t e = top >> 23;  // biased exponent
-  const int shift = top == 0 ? 0 : int(e < kLow ? kLow : kHigh) - int(e);
-  if (threadIdx.x == 0) undo[m] = __uint_as_float((uint32_t(127 - shift) << 23) | (all & 4u ? 0x80000000u : 0u));
+  for (int w = 0; w < waves; ++w)
+    top = max(top & 0x7FFFFFFFu, seen[w] & 0x7FFFFFFFu) | ((top | seen[w]) & 0x80000000u);
+  const uint32_t e = (top & 0x7FFFFFFFu) >> 23;  // biased exponent
+  const int shift = (top & 0x7FFFFFFFu) == 0 ? 0 : e < kLow ? int(kLow - e) : e > kHigh ? int(kHigh) - int(e) : 0;
+  if (first) undo[m] = __uint_as_float((uint32_t(127 - shift) << 23) | (top & 0x80000000u));
   if (shift != 0) split_row(__uint_as_float(uint32_t(127 + shift) << 23), std::false_type{});
 }
 
@@ -680,13 +697,19 @@ hipError_t launch_linear_f32_gemm(const LinearArgs& a, hipStream_t stream, bool*
   g.undo = undo;
   g.partials = reinterpret_cast<float*>(ws + p.pieces + p.sums + p.undo);
   const float* x = static_cast<const float*>(a.x);
-  const dim3 sgrid{unsigned(a.M)}, sblock{unsigned(std::min<int64_t>(kSplitThreads, (a.K / 8 + 63) / 64 * 64))};
+  // Up to 128 rows: several workgroups per row, of 256 threads where four rounds of them cover it.
+  const int64_t chunks = a.K / 8;
+  const int64_t threads = std::min<int64_t>(a.M <= 128 && chunks <= 1024 ? 256 : kSplitThreads, (chunks + 63) / 64 * 64);
+  const int64_t rounds = (chunks + threads - 1) / threads;
+  int parts = 1;
+  while (a.M <= 128 && 2 * parts <= rounds) parts *= 2;
+  const dim3 sgrid(unsigned(a.M), unsigned(parts)), sblock{unsigned(threads)};
   if (a.ldx % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0)
     hipLaunchKernelGGL(split_tiles_kernel<true>, sgrid, sblock, 0, stream, x, a.ldx, p.mpad,
-                       int(a.K / kBK), ws, sums, undo);
+                       int(a.K / kBK), parts, ws, sums, undo);
   else
     hipLaunchKernelGGL(split_tiles_kernel<false>, sgrid, sblock, 0, stream, x, a.ldx, p.mpad,
-                       int(a.K / kBK), ws, sums, undo);
+                       int(a.K / kBK), parts, ws, sums, undo);
   if (a.fmt == kNibble)
     p.tt == 2 ? launch_tt<2, kNibble>(a, g, stream) : launch_tt<1, kNibble>(a, g, stream);
   else
