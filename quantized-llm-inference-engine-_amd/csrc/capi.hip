@@ -536,10 +536,13 @@ int describe_cache(llmopt::KvWriteArgs& a, void* key_cache, void* value_cache, i
 // With heads of 128 a CU holds one workgroup of eight waves (157 registers, 187 with the rotary step),
 // so a grid of 257 - 511 of them runs in two rounds, the second nearly empty. There the split stays
 // at one round's 256 workgroups, and more than 256 pairs take workgroups of four waves, of which two share
-// a CU. Measured (MI355X, 32 / 8 heads; us against the split rounded up): 24 sequences of 320 - 640 tokens
-// 13.7 / 20.7, of 2048 - 4096 72 / 81, 9 of 1024 - 2048 18.9 / 26.5, 48 of 320 - 640 26.6 / 29.4 (28.2 / 30.1
-// with the rotary step). Past 512 pairs smaller workgroups lost (640 pairs 41.3 / 39.9, 1280 71 / 66), and
-// heads of 64 (at most 124 registers) fit two workgroups of eight waves per CU, a whole grid of up to 511.
+// a CU, over tables of up to 64 tiles (1024 tokens). Measured (MI355X, 32 / 8 heads; us against the split
+// rounded up): 24 sequences of 320 - 640 tokens 13.7 / 20.7, of 2048 - 4096 72 / 81, 9 of 1024 - 2048 18.9 / 26.5;
+// four waves against eight, 33 / 48 / 63 sequences of 150 - 300 11.6 / 13.6 / 14.6 against 14.3 / 16.9 / 17.6, of
+// 450 - 900 23.8 / 28.2 / 32.2 against 25.3 / 30.3 / 33.2. Longer contexts want every wave: level at 600 - 1200
+// (28.7 / 35.1 / 42.3 against 27.6 / 37.0 / 41.8), of 2000 - 4000 127 / 142 / 157 against 112 / 132 / 160. Past 512
+// pairs smaller workgroups lost (640 pairs 41.3 / 39.9, 1280 71 / 66), and heads of 64 (at most 124
+// registers) fit two workgroups of eight waves per CU, a whole grid of up to 511.
 struct DecodePlan {
   int splits;
   int waves;
@@ -556,7 +559,7 @@ DecodePlan plan_decode(int64_t num_seqs, int64_t kv_heads, int64_t head_dim, int
   const int wmax = group >= 16 ? 4 : 8;
   const bool wide = head_dim == 128;
   int waves = 1;
-  while (waves < wmax && waves < parts && !(wide && waves == 4 && pairs > 256)) waves *= 2;
+  while (waves < wmax && waves < parts && !(wide && waves == 4 && pairs > 256 && tiles <= 64)) waves *= 2;
   int64_t splits = (parts + waves - 1) / waves;
   if (wide && splits > 1 && splits * waves * pairs > 2048) splits = std::max<int64_t>(1, 2048 / (waves * pairs));
   if (splits > 64) splits = 64;

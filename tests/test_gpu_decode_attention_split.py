@@ -1,10 +1,10 @@
 """Decode attention at the edges of its work split, against the oracle's float64 attention.
 
 With heads of 128 the grid of (sequence, KV head) pairs times context splits stays within one workgroup of
-eight waves per CU (256 of them), and more than 256 pairs take four waves per workgroup; heads of 64 split
-as their smaller register count allows. Bounds as for every decode attention output: the probabilities
-are rounded to the cache dtype (as the reference's are) and the output once to the query dtype, 1e-2 for
-bf16 and 2e-3 for fp16."""
+eight waves per CU (256 of them), and more than 256 pairs take four waves per workgroup up to a table of
+1024 tokens; heads of 64 split as their smaller register count allows. Bounds as for every decode attention
+output: the probabilities are rounded to the cache dtype (as the reference's are) and the output once to
+the query dtype, 1e-2 for bf16 and 2e-3 for fp16."""
 
 from __future__ import annotations
 
@@ -21,11 +21,13 @@ DEV = torch.device("cuda:0")
 TOL = {torch.bfloat16: 1e-2, torch.float16: 2e-3}
 
 # (sequences, heads, kv_heads, head_dim, longest context): pairs of 128, 129, 160 and 255 - 257, 264,
-# 511 and 512; several splits capped (72 and 96 pairs over long contexts); 16 query heads per KV head.
+# 511 and 512; several splits capped (72 and 96 pairs over long contexts); 16 query heads per KV head;
+# 257 and 264 pairs on both sides of a table of 64 tiles.
 CASES = [
     (16, 16, 8, 128, 300), (129, 1, 1, 128, 300), (20, 32, 8, 128, 290), (255, 2, 1, 128, 150), (32, 8, 8, 128, 300),
     (257, 4, 1, 128, 150), (33, 32, 8, 128, 290), (73, 14, 7, 128, 150), (64, 8, 8, 128, 150), (9, 32, 8, 128, 1100),
     (12, 8, 8, 128, 1030), (20, 128, 8, 128, 290), (33, 128, 8, 128, 290), (20, 16, 8, 64, 290), (33, 16, 8, 64, 290),
+    (257, 4, 1, 128, 1024), (257, 4, 1, 128, 1025), (33, 32, 8, 128, 1040),
 ]
 
 
