@@ -4,7 +4,7 @@
 // kernel argument block and picks the kernel: the decode kernels for M <= 32, the MFMA
 // register-dequant GEMM (split over K on small grids) above, from 1024 tokens the weight
 // dequantized into the workspace and hipBLASLt's dense GEMM, for fp32 activations past one decode pass
-// the GEMM over exact bf16 pieces (the dense product for small weights and the shapes that it does not take), the
+// the GEMM over exact bf16 pieces (the dense product for the shapes that it does not take), the
 // LDS-dequant GEMM for the shapes the register-dequant one does not take, and the generic kernel
 // for shapes, alignments or dtypes the fast kernels do not take. Error text is kept per host
 // thread.
@@ -129,15 +129,6 @@ bool dense_first(int64_t M, int64_t N, int64_t K, int act, const void* workspace
          workspace_bytes >= llmopt::dense_workspace_bytes(N, K, act);
 }
 
-// fp32 weights so small that the two-pass path's launches (dequantize, product) end before the GEMM's three
-// (split, GEMM, reduction) have begun in earnest. Measured (MI355X, groups of 64, us GEMM / dense): 1024 x 1024 at
-// 65, 128, 500, 1000 and 1536 tokens 16.2 / 10.9, 17.5 / 11.3, 22.5 / 19.1, 28.7 / 27.6, 32.2 / 35.3; 256 x 4096 at 65
-// and 1000 18.3 / 13.8, 31.1 / 27.1; 1536 x 1024 at 65 and 128 16.9 / 12.5, 17.6 / 14.6, slower from 130 on; 1024 x
-// 2816 at 65 and 128 19.2 / 18.5, 21.4 / 20.1, where the GEMM's smaller error (a fifth) is kept.
-bool small_for_dense(int64_t M, int64_t N, int64_t K) {
-  return (M <= 1024 && N * K <= int64_t(1) << 20) || (M <= 128 && N * K <= int64_t(3) << 19);
-}
-
 // Dispatch shared by llmopt_q_linear_ex and llmopt_q_linear_swiglu. With the SwiGLU epilogue,
 // `y` is [M, N/2]; kernels that cannot apply it themselves write the full [M, N] product into
 // the workspace and a combining kernel finishes.
@@ -214,8 +205,7 @@ int run_linear(const void* x, int64_t M, int64_t K, int64_t ldx, const void* qwe
     return hip_status(llmopt::launch_swiglu_combine(t, N, y, ldy, M, N, act_dtype, s), "swiglu launch");
   }
 
-  if (act_dtype == LLMOPT_DTYPE_F32 && algo == LLMOPT_ALGO_AUTO && M >= llmopt::f32_gemm_min_tokens(a.group) &&
-      !(small_for_dense(M, N, K) && dense_first(M, N, K, act_dtype, a.workspace, a.workspace_bytes))) {
+  if (act_dtype == LLMOPT_DTYPE_F32 && algo == LLMOPT_ALGO_AUTO && M >= llmopt::f32_gemm_min_tokens(a.group)) {
     // fp32 activations past one decode pass: the GEMM over exact bf16 pieces.
     err = llmopt::launch_linear_f32_gemm(a, s, &fits);
     if (fits) return hip_status(err, "fp32 linear");

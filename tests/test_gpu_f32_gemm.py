@@ -12,8 +12,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from llmopt.kernels import _lib, ops
-from llmopt.kernels._lib import ALGO_DENSE
+from llmopt.kernels import ops
 from llmopt.quantization import QuantizedTensor
 
 pytestmark = pytest.mark.gpu
@@ -49,22 +48,6 @@ def _weight(n, k, bits, group, symmetric, seed, zeros="int"):
     return qt, w, mag if zeros != "int" else w.abs()
 
 
-def _gemm(x, qt, bias):
-    """The product with a workspace a little short of the dense path's, which small weights would take."""
-    lib = _lib.load_library()
-    f32 = _lib.DTYPE_CODES[torch.float32]
-    (n, k), m = qt.shape, x.shape[0]
-    size = lib.llmopt_q_linear_dense_workspace(n, k, f32) - 256
-    assert x.stride(1) == 1
-    y, ws = torch.empty(m, n, device=DEV), torch.empty(size, dtype=torch.uint8, device=DEV)
-    _lib.call(lib.llmopt_q_linear(x.data_ptr(), m, k, x.stride(0), qt.qweight.data_ptr(), qt.qweight.shape[1],
-                                  qt.scales.data_ptr(), None if qt.symmetric else qt.zeros.data_ptr(),
-                                  None if bias is None else bias.data_ptr(), y.data_ptr(), n, n, f32, qt.bits,
-                                  qt.group_size, int(qt.symmetric), int(qt.qweight.dtype == torch.int8),
-                                  ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream), "llmopt_q_linear")
-    return y
-
-
 def _check(y, x, w, mag, group, bias=None):
     ref = x.double() @ w.t()
     k = x.shape[1]
@@ -89,7 +72,7 @@ def test_edges_of_tiles(shape, m):
     g = torch.Generator().manual_seed(m)
     x = torch.randn(m, k, generator=g).to(DEV)
     bias = torch.randn(n, generator=g).to(DEV) if m % 2 else None
-    _check(_gemm(x, qt, bias), x, w, mag, group, bias)
+    _check(ops.quant_linear(x, qt, bias, torch.float32), x, w, mag, group, bias)
 
 
 @pytest.mark.parametrize("zeros", ["fraction", "far"])
@@ -99,7 +82,7 @@ def test_zero_points_off_the_integer_range(zeros, bits, group):
     # through the sums of x.
     qt, w, mag = _weight(300, 1024, bits, group, False, seed=5, zeros=zeros)
     x = torch.randn(70, 1024, generator=torch.Generator().manual_seed(6)).to(DEV)
-    _check(_gemm(x, qt, None), x, w, mag, group)
+    _check(ops.quant_linear(x, qt, None, torch.float32), x, w, mag, group)
 
 
 def test_unaligned_rows_and_wide_magnitudes():
@@ -108,7 +91,7 @@ def test_unaligned_rows_and_wide_magnitudes():
     g = torch.Generator().manual_seed(8)
     base = torch.randn(m, k + 3, generator=g) * torch.exp2(torch.randint(-40, 40, (m, 1), generator=g).float())
     x = base.to(DEV)[:, 1 : k + 1]  # rows off 16-byte alignment, stride k + 3
-    _check(_gemm(x, qt, None), x, w, mag, 64)
+    _check(ops.quant_linear(x, qt, None, torch.float32), x, w, mag, 64)
 
 
 def test_infinities_and_nan_match_the_dense_product():
@@ -117,7 +100,7 @@ def test_infinities_and_nan_match_the_dense_product():
     x = torch.randn(m, k, generator=torch.Generator().manual_seed(10)).to(DEV)
     x[3, 17], x[4, 200], x[5, 0] = float("inf"), float("-inf"), float("nan")
     x[6, 9] = 3.0e38  # finite, rounds to infinity in bf16, and overflows times the integer weight
-    y = _gemm(x, qt, None)
+    y = ops.quant_linear(x, qt, None, torch.float32)
     ref = x.double() @ w.t()
     assert torch.equal(torch.isnan(y), torch.isnan(ref))
     assert torch.equal(torch.isposinf(y), torch.isposinf(ref))
@@ -134,14 +117,14 @@ def test_infinities_with_remainders_of_zero_points(m, n, k, bits, group, zeros):
     # weight of exactly zero, or infinities of both signs, make a NaN. Other rows keep their values.
     qt, w, mag = _weight(n, k, bits, group, False, seed=17, zeros=zeros)
     x = torch.randn(m, k, generator=torch.Generator().manual_seed(18)).to(DEV)
-    y0 = _gemm(x, qt, None)
+    y0 = ops.quant_linear(x, qt, None, torch.float32)
     _check(y0, x, w, mag, group)
     inf = float("inf")
     for row, at in ((3, {17: inf}), (4, {200: -inf}), (5, {0: float("nan")}), (6, {9: inf, 70: inf}),
                     (7, {8: inf, 9: -inf}), (m - 1, {k - 1: inf, 3: 2.0e38})):
         for c, v in at.items():
             x[row, c] = v
-    y, ref = _gemm(x, qt, None), x.double() @ w.t()
+    y, ref = ops.quant_linear(x, qt, None, torch.float32), x.double() @ w.t()
     assert torch.equal(torch.isnan(y), torch.isnan(ref))
     assert torch.equal(torch.isposinf(y), torch.isposinf(ref)) and torch.equal(torch.isneginf(y), torch.isneginf(ref))
     rest = [i for i in range(m - 1) if i not in (3, 4, 5, 6, 7)]
@@ -161,7 +144,7 @@ def test_the_whole_range_of_fp32(m, n, k, bits, group, symmetric):
     size = torch.linspace(-140, 126, m).round()
     x = (x.double() * torch.exp2(size.double())[:, None]).float().to(DEV)
     bound = (x.double().abs() @ mag.t()) * ((3 * group + k / group + 4) * 2.0**-23 * (1 + 2.0**-7)) + 2.0**-148
-    y, ref = _gemm(x, qt, None).double(), x.double() @ w.t()
+    y, ref = ops.quant_linear(x, qt, None, torch.float32).double(), x.double() @ w.t()
     fits = ref.abs() < 3.4e38  # else the dense product is infinite as well
     assert bool(((y - ref).abs()[fits] <= bound[fits]).all()) and bool(torch.isinf(y[ref.abs() > 3.5e38]).all())
 
@@ -185,6 +168,8 @@ def test_swiglu_of_large_and_small_rows():
 
 def test_partial_workspace_keeps_the_decode_passes():
     # Enough for the decode kernels' pieces and not for the GEMM's tiles: the chunks run as before.
+    from llmopt.kernels import _lib
+
     lib = _lib.load_library()
     n, k, m = 512, 2048, 40
     qt, w, mag = _weight(n, k, 4, 64, True, seed=11)
@@ -199,20 +184,6 @@ def test_partial_workspace_keeps_the_decode_passes():
                                  torch.cuda.current_stream().cuda_stream)
         assert rc == 0, lib.llmopt_q_last_error()
         assert float((y - full).abs().max()) <= 1e-5 * float(full.abs().max())
-
-
-@pytest.mark.parametrize("n,k,last", [(1024, 1024, 1024), (256, 4096, 1024), (1536, 1024, 128), (1024, 2816, None)])
-def test_small_weights_take_the_dense_product(n, k, last):
-    # From 65 tokens, up to 2^20 weights and 1024 tokens or 3 * 2^19 and 128: the pinned dense call's bits; beyond
-    # either, the GEMM's.
-    qt, w, _ = _weight(n, k, 4, 64, True, seed=19)
-    for m in (64, 65, 128, 129, 1024, 1025):
-        x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(DEV)
-        y = ops.quant_linear(x, qt, None, torch.float32)
-        other = ops.quant_linear(x, qt, None, torch.float32, algo=ALGO_DENSE)
-        dense = last is not None and 65 <= m <= last
-        assert torch.equal(y, other if dense else _gemm(x, qt, None)) and not torch.equal(other, _gemm(x, qt, None))
-        assert float((y.double() - x.double() @ w.t()).abs().max()) <= 2e-5 * float(y.abs().max())
 
 
 @pytest.mark.parametrize("m,inter,k", [(17, 128, 128), (33, 100, 1024), (65, 516, 2048), (500, 1024, 512), (300, 14336, 256)])
