@@ -28,7 +28,7 @@
 // owns 256 output features x 32 TT tokens; each wave takes 64 features and every token, so an LDS
 // fragment read (the A operand, 32 tokens x 16 k) feeds two MFMAs and a weight fragment (the B operand,
 // one 32-bit word of packed codes per lane) is dequantized by exactly one wave and feeds 3 TT. Two
-// workgroups share a CU (72 KB of LDS and at most 224 registers each), which fills one's barriers, folds and
+// workgroups share a CU (72 KB of LDS and at most 229 registers each), which fills one's barriers, folds and
 // dequantization with the other's MFMAs.
 #include <algorithm>
 #include <type_traits>

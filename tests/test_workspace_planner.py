@@ -18,7 +18,8 @@ Llama-3-8B projections without a GPU (no kernel is launched):
 * the prefill GEMM's own plan above 64 tokens;
 * from 1024 tokens the two-pass path: the dense weight in the compute dtype (256-byte aligned)
   and 32 MiB for hipBLASLt, or the fused plan's bytes where those are more (what runs when
-  hipBLASLt has no algorithm); fp32 activations from 65 tokens.
+  hipBLASLt has no algorithm); fp32 activations from 65 tokens, also where the GEMM over pieces
+  takes the call.
 """
 
 from __future__ import annotations
@@ -153,7 +154,8 @@ def test_long_batches_take_the_two_pass_path(lib, m):
         assert sw == -(-m * n * 2 // 256) * 256 + _dense(n, k, 2)
 
 
-def test_fp32_takes_the_two_pass_path_from_65_tokens(lib):
+def test_fp32_asks_for_the_two_pass_path_from_65_tokens(lib):
+    # The GEMM over pieces takes most of these calls with less, but a weight off 16 bytes needs the dense one.
     f32 = _lib.DTYPE_CODES[torch.float32]
     n, k = GATE_UP
     assert lib.llmopt_q_linear_workspace_ex(64, n, k, 4, 64, f32) < _dense(n, k, 4)
