@@ -45,7 +45,8 @@ cpu_baseline   the reference's host sequence (dequantize once, cache the dense w
 Every single-projection timing (roofline, prefill, shapes, bits_sweep) rotates over at least
 512 MiB of that projection's own weight copies.
 
-Modes: default prints the JSON line. `--e2e-only` runs only the end-to-end generation (for a
+Modes: default prints the JSON line; the tables (shapes, bits_sweep, engine_config, cpu_baseline's
+`configs`) go to stderr after `# details`, or to the file that `--details` names. `--e2e-only` runs only the end-to-end generation (for a
 kernel trace of it). `--pmc-workload` runs only the dominant kernel and a
 256 MiB copy (for `rocprofv3 --pmc FETCH_SIZE` / `--pmc WRITE_SIZE`); `--traffic-from DIR`
 turns two such rocprofv3 CSV outputs into profiles/traffic_decode_gate_up_m1.json;
@@ -53,7 +54,7 @@ turns two such rocprofv3 CSV outputs into profiles/traffic_decode_gate_up_m1.jso
 `--trace-kernels CSV` per kernel and grid.
 
 Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-shapes] [--no-cpu]
-       [--no-prefill] [--no-e2e] [--e2e-only]
+       [--no-prefill] [--no-e2e] [--e2e-only] [--details FILE]
 """
 
 from __future__ import annotations
@@ -103,6 +104,8 @@ def parse_args() -> argparse.Namespace:
     p.add_argument("--no-e2e", action="store_true", help="skip the end-to-end Llama-3-8B generation")
     p.add_argument("--e2e-only", action="store_true", help="only the end-to-end generation (for profiling)")
     p.add_argument("--cpu-seconds", type=float, default=15.0)
+    p.add_argument("--details", type=str, default=None,
+                   help="write the per-shape, bit-width, engine and CPU tables to this file instead of stderr")
     p.add_argument("--pmc-workload", action="store_true", help="only the dominant kernel + a copy")
     p.add_argument("--pmc-prefill", action="store_true",
                    help="only gate_up at M = 8192, two-pass and fused GEMM, three calls each (for --pmc)")
@@ -372,8 +375,25 @@ def main() -> int:
         result["engine_config"] = engine_config(torch, ops)
     if not args.no_cpu:
         result["cpu_baseline"] = cpu_baseline(torch, base, args.m, args.cpu_seconds, gptq)
-    print(json.dumps(result), flush=True)
+    line, details = split_result(result)
+    if args.details:
+        Path(args.details).write_text(json.dumps(details) + "\n")
+    else:
+        print("# details " + json.dumps(details), file=sys.stderr, flush=True)
+    print(json.dumps(line), flush=True)
     return 0
+
+
+def split_result(result: dict) -> tuple[dict, dict]:
+    """The JSON line -- the headline and one figure per block, a few kilobytes that a reader with a
+    bounded tail of the output still gets whole -- and the long tables (per shape, bit width and CPU
+    configuration), which go to stderr or to the file that ``--details`` names."""
+    line = dict(result)
+    details = {key: line.pop(key) for key in ("shapes", "bits_sweep", "engine_config") if key in line}
+    if isinstance(line.get("cpu_baseline"), dict) and "configs" in line["cpu_baseline"]:
+        line["cpu_baseline"] = {k: v for k, v in line["cpu_baseline"].items() if k != "configs"}
+        details["cpu_baseline_configs"] = result["cpu_baseline"]["configs"]
+    return line, details
 
 
 def _code_only(text: str) -> str:
